@@ -26,7 +26,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 OBJ = os.path.join(HERE, "_obj")
 
-HIP_SOURCES = ["capi.hip", "flatquant_quant.hip", "int4_gemm.hip", "int4_gemm_f6.hip", "dequant.hip", "layout.hip", "w4a4_linear.hip"]
+HIP_SOURCES = ["capi.hip", "flatquant_quant.hip", "flatquant_tile_f16.hip", "flatquant_tile_bf16.hip", "int4_gemm.hip", "int4_gemm_f6.hip", "dequant.hip", "layout.hip", "w4a4_linear.hip"]
 LIB_NAME = "libquant_ops_hip.so"
 TORCH_LIB_NAME = "_quant_ops_torch.so"
 # microbenchmarks of the hardware ceilings (bench.py --ceilings), a library of its own
@@ -52,9 +52,11 @@ HIP_FLAGS = [
 # quantize kernels also take their first 16 argument dwords preloaded into
 # SGPRs (no scalar load before the first DMA issue: 1-2% on launches of a few
 # microseconds); the GEMM measured no gain from it.
+_QUANTIZE_FLAGS = ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 FILE_FLAGS = {
-    "flatquant_quant.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1",
-                            "-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    "flatquant_quant.hip": _QUANTIZE_FLAGS,
+    "flatquant_tile_f16.hip": _QUANTIZE_FLAGS,
+    "flatquant_tile_bf16.hip": _QUANTIZE_FLAGS,
 }
 
 

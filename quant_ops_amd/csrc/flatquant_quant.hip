@@ -14,12 +14,14 @@
 //                       workgroups per CU (112 x 128 and 64 x 128).
 //  * fq_duo_kernel    — a pair of waves per token, the same shapes (kept for
 //                       cross-checks: QO_ROUTE_FQ_NO_FEW routes N = 128 to it).
-//  * fq_mfma_kernel   — D in {fp16, bf16}, the listed shapes: M up to 176 zero-padded
-//                       to 16 MB, N even up to 256 zero-padded to 32 NP.
+//  * fq_mfma_kernel   — D in {fp16, bf16}, the listed shapes: M up to 128 zero-padded
+//                       to 16 MB, N a multiple of 8 up to 256 zero-padded to 32 NP.
 //                       Both contractions on v_mfma_f32_16x16x32_{f16,bf16}; X is
 //                       streamed into LDS by LDS-DMA one token group ahead (two
 //                       stages, one where two do not fit); L is resident in VGPRs
 //                       or LDS, R in VGPRs.
+//  * fq_tile_kernel   — (flatquant_tile.h) fp16 / bf16, every other shape with N
+//                       even up to 256 and M up to 176.
 //  * fq_generic_kernel — any M, N, D in {fp32, fp16, bf16}; VALU fp32 FMA with the
 //                       same rounding points. Used for shapes the MFMA kernels
 //                       do not cover (and for fp32 inputs), X and Z in LDS.
@@ -33,50 +35,14 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "common.h"
+#include "flatquant_common.h"
 
 namespace qo {
 
-// ---------------------------------------------------------------------------
-// Scale and code, shared by both kernels.
-// ---------------------------------------------------------------------------
-
-// Per-token scale from the raw (unrounded) fp32 extremes of Y. Rounding to D is
-// monotonic, so rnd_D(max y) == max rnd_D(y): this is amax/amin of the D tensor
-// (ops.py:108-109), then maximum(|rnd(min*c)|, rnd(max*c)) (ops.py:112), then
-// rnd(./7) clamped below by rnd_D(1e-8) (ops.py:113).
+// fq_tile_kernel (flatquant_tile.h): false where it has no instance for the shape.
 template <class DT>
-__device__ inline float fq_scale(float ymax_raw, float ymin_raw, float clip) {
-  const float hi = DT::round(ymax_raw);
-  const float lo = DT::round(ymin_raw);
-  const float t_lo = DT::round(lo * clip);
-  const float t_hi = DT::round(hi * clip);
-  const float bound = fmaxf(fabsf(t_lo), t_hi);
-  const float s = DT::round(opaque(bound) / 7.0f);
-  return fmaxf(s, DT::round(1e-8f));
-}
-
-// The same scale from max |Y| of the D-rounded Y, valid for clip > 0:
-// rounding to nearest even is sign-symmetric and monotonic, so
-// max(|rnd(rnd(min) c)|, rnd(rnd(max) c)) = rnd(max |rnd(y)| c).
-template <class DT>
-__device__ inline float fq_scale_abs(float amax, float clip) {
-  const float bound = DT::round(amax * clip);
-  const float s = DT::round(opaque(bound) / 7.0f);
-  return fmaxf(s, DT::round(1e-8f));
-}
-
-// Code of one element from its D-rounded quotient t = rnd_D(y / s):
-// clamp(round_half_even(t), -8, 7) (ops.py:117). A NaN quotient (0/0 when an
-// fp16 token's scale rounds to 0) becomes 0 through the reference's int8 cast
-// and nibble 0 (code -8) through its uint8 cast before packing (ops.py:122);
-// both are reproduced here.
-template <bool PACK>
-__device__ inline int fq_code_from_quot(float t) {
-  if (t != t) return PACK ? -8 : 0;
-  const float c = fminf(fmaxf(t, -8.0f), 7.0f);
-  return (int)__builtin_rintf(c);
-}
+bool launch_tile(const void* x, int64_t tokens, int64_t x_ld, const void* left, const void* right, int M, int N,
+                 float clip, int pack, void* out_codes, float* out_scales, hipStream_t stream);
 
 // ---------------------------------------------------------------------------
 // Generic kernel: one block of BT threads per token (grid-stride over tokens).
@@ -368,264 +334,16 @@ fq_generic_big_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int6
 // only has to agree between the A and B operands.
 // ---------------------------------------------------------------------------
 
-template <class DT>
-struct MfmaOps;
-
-// V: 8-element operands of the 16x16x32 MFMA. An odd trailing 16-deep slab of
-// the second product (M / 16 odd) is a zero-padded 32-deep slab: elements 0..3
-// of lane group g hold k = 4g .. 4g+3 (the rows of Z's accumulator), elements
-// 4..7 of both operands are zero, which leaves the MFMA's sum unchanged. (The
-// 16x16x16 MFMA gave wrong results in that role on gfx950.)
-template <>
-struct MfmaOps<F16T> {
-  using V = v8h;
-  __device__ static inline v4f mfma(V a, V b, v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-
-template <>
-struct MfmaOps<BF16T> {
-  using V = v8bf;
-  __device__ static inline v4f mfma(V a, V b, v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-
-// Epilogue on packed pairs. A lane's Y values come in pairs (MFMA block h = 0
-// and 1 at the same accumulator row r) that belong in nibbles r and r + 4 of
-// one output word, so each pair is kept as two 16-bit D values in one VGPR
-// (rounding point 2 for both with one v_cvt_pk). Quantizing a pair:
-//   a = clamp(y * rcp, -8, 7) in float32   (clamp commutes with the roundings
-//                                           below because -8 and 7 are D values)
-//   t = rnd_D(a)                           (one v_cvt_pk for the pair)
-//   t + magic                              (round half to even to an integer)
-// The magic constant leaves q + 8 in the low bits of each result; shifting the
-// pair's bits by 4r and adding puts both codes in place, and the constant bits
-// the magic leaves above the codes add up to kJunk, removed once per word.
-// y * rcp stands in for the fallback's y / s (IEEE): the two differ only when
-// the quotient lies within a few float32 ulps of a rounding boundary of D.
-template <class DT>
-struct FqEpi;
-
-template <>
-struct FqEpi<F16T> {
-  __device__ static inline uint32_t pack(float a, float b) {
-    const v2h h = {(_Float16)opaque(a), (_Float16)opaque(b)};
-    return __builtin_bit_cast(uint32_t, h);
-  }
-  // The same rounding of two MFMA accumulator values. An MFMA result has no
-  // product for the compiler to fuse into the conversion, so no opaque() is
-  // needed (which would copy accumulators that are read again for the absmax).
-  __device__ static inline uint32_t pack_acc(float a, float b) {
-    const v2h h = {(_Float16)a, (_Float16)b};
-    return __builtin_bit_cast(uint32_t, h);
-  }
-  __device__ static inline float lo(uint32_t p) { return (float)__builtin_bit_cast(v2h, p)[0]; }
-  __device__ static inline float hi(uint32_t p) { return (float)__builtin_bit_cast(v2h, p)[1]; }
-  // fp16: 1544 = 1536 + 8 has a unit ulp, so t + 1544 is the integer 1536 + q + 8,
-  // bits 0x6600 + (q + 8); both halves are handled by one v_pk_add_f16.
-  __device__ static inline void accumulate(uint32_t& word, uint32_t p, float rcp, int r) {
-    const float a0 = __builtin_amdgcn_fmed3f(mul_f16lo(p, rcp), -8.0f, 7.0f);
-    const float a1 = __builtin_amdgcn_fmed3f(mul_f16hi(p, rcp), -8.0f, 7.0f);
-    v2h t = __builtin_bit_cast(v2h, pack(a0, a1));
-    const v2h magic = {(_Float16)1544.0f, (_Float16)1544.0f};
-    t = t + magic;
-    word += __builtin_bit_cast(uint32_t, t) << (4 * r);
-  }
-  static constexpr uint32_t kJunk =
-      0x66006600u + (0x66006600u << 4) + (0x66006600u << 8) + (0x66006600u << 12);
-
-  // Packed word of four pairs (nibbles r and r + 4 from pair r), clamping the
-  // rounded pair instead of the float32 quotients: rounding is monotonic and
-  // -8, 7 are fp16 values, so clamp(rnd(a)) = rnd(clamp(a)). One packed min per
-  // pair, plus one packed max when a quotient can round below -8.5 (LOW).
-  template <bool LOW>
-  __device__ static inline uint32_t word4(const uint32_t (&p)[4], float rcp) {
-    const v2h seven = {(_Float16)7.0f, (_Float16)7.0f};
-    const v2h minus8 = {(_Float16)-8.0f, (_Float16)-8.0f};
-    const v2h magic = {(_Float16)1544.0f, (_Float16)1544.0f};
-    uint32_t word = 0u - kJunk;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      v2h t = __builtin_bit_cast(v2h, pack(mul_f16lo(p[r], rcp), mul_f16hi(p[r], rcp)));
-      t = __builtin_elementwise_min(t, seven);
-      if (LOW) t = __builtin_elementwise_max(t, minus8);
-      t = t + magic;
-      word += __builtin_bit_cast(uint32_t, t) << (4 * r);
-    }
-    return word;
-  }
-
-  // Running extremes of rounded Y pairs, two pairs per step (v_pk_maximum3 /
-  // v_pk_minimum3), and max |y| from them as a 16-bit pattern.
-  struct Amax {
-    v2h hi = {(_Float16)-INFINITY, (_Float16)-INFINITY};
-    v2h lo = {(_Float16)INFINITY, (_Float16)INFINITY};
-  };
-  __device__ static inline void track2(Amax& a, uint32_t p0, uint32_t p1) {
-    const v2h y0 = __builtin_bit_cast(v2h, p0), y1 = __builtin_bit_cast(v2h, p1);
-    a.hi = __builtin_elementwise_maximum(__builtin_elementwise_maximum(a.hi, y0), y1);
-    a.lo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(a.lo, y0), y1);
-  }
-  __device__ static inline uint32_t amax_bits(const Amax& a) {
-    const uint32_t m = pk_absmax16(pk_absmax16(0u, __builtin_bit_cast(uint32_t, a.hi)),
-                                   __builtin_bit_cast(uint32_t, a.lo));
-    return max(m & 0xFFFFu, m >> 16);
-  }
-};
-
-template <>
-struct FqEpi<BF16T> {
-  __device__ static inline uint32_t pack(float a, float b) {
-    const v2bf h = {(__bf16)opaque(a), (__bf16)opaque(b)};
-    return __builtin_bit_cast(uint32_t, h);
-  }
-  __device__ static inline uint32_t pack_acc(float a, float b) {
-    const v2bf h = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(uint32_t, h);
-  }
-  __device__ static inline float lo(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
-  __device__ static inline float hi(uint32_t p) { return __builtin_bit_cast(float, p & 0xFFFF0000u); }
-  // bf16: rounded pair back to float32, then + 12582920 = 1.5 * 2^23 + 8 leaves
-  // bits 0x4B400000 + (q + 8). The high element is shifted by 16 + 4r, which
-  // drops all of 0x4B400000; the low element's constant part sums to kJunk.
-  __device__ static inline void accumulate(uint32_t& word, uint32_t p, float rcp, int r) {
-    const float a0 = __builtin_amdgcn_fmed3f(lo(p) * rcp, -8.0f, 7.0f);
-    const float a1 = __builtin_amdgcn_fmed3f(hi(p) * rcp, -8.0f, 7.0f);
-    const uint32_t t = pack(a0, a1);
-    const float f0 = lo(t) + 12582920.0f;
-    const float f1 = hi(t) + 12582920.0f;
-    word += __builtin_bit_cast(uint32_t, f0) << (4 * r);
-    word += __builtin_bit_cast(uint32_t, f1) << (16 + 4 * r);
-  }
-  static constexpr uint32_t kJunk =
-      0x4B400000u + (0x4B400000u << 4) + (0x4B400000u << 8) + (0x4B400000u << 12);
-
-  // Packed word of four pairs (the float32 clamp covers both bounds).
-  template <bool LOW>
-  __device__ static inline uint32_t word4(const uint32_t (&p)[4], float rcp) {
-    uint32_t word = 0u - kJunk;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) accumulate(word, p[r], rcp, r);
-    return word;
-  }
-
-  // Code byte B of d from a rounded quotient t (a bf16 value in a float32
-  // register, -8.5 <= t < 7.5): one SDWA add of 12582920 = 1.5 * 2^23 + 8,
-  // whose float32 sum has a unit ulp, so it rounds t + 8 half to even, which
-  // is rint(t) + 8 (8 is even), and leaves that integer (0 .. 15) in the
-  // low byte of its bits; dst_sel writes that byte into byte B of d, the
-  // other bytes kept (FIRST: cleared). A NaN t (its float32 low half zero)
-  // gives byte 0, as v_cvt_pk_u8_f32 of t + 8 does.
-  template <int B, bool FIRST>
-  __device__ static inline void code_byte(uint32_t& d, float t, float magic) {
-    static_assert(!FIRST || B == 0, "the first byte of a word clears the rest");
-#define QO_CODE_BYTE(SEL, UNUSED, C)                                                                         \
-  asm("v_add_f32_sdwa %0, %1, %2 dst_sel:" SEL " dst_unused:" UNUSED " src0_sel:DWORD src1_sel:DWORD"     \
-      : C(d)                                                                                                \
-      : "v"(t), "v"(magic))
-    if constexpr (FIRST) QO_CODE_BYTE("BYTE_0", "UNUSED_PAD", "=v");
-    else if constexpr (B == 1) QO_CODE_BYTE("BYTE_1", "UNUSED_PRESERVE", "+v");
-    else if constexpr (B == 2) QO_CODE_BYTE("BYTE_2", "UNUSED_PRESERVE", "+v");
-    else QO_CODE_BYTE("BYTE_3", "UNUSED_PRESERVE", "+v");
-#undef QO_CODE_BYTE
-  }
-
-  // The packed word of four pairs from rounded quotients t[i] (code i):
-  // even codes in the bytes of ev, odd codes in the bytes of od, and
-  // ev | od << 4 puts code i in nibble i.
-  __device__ static inline uint32_t word_from_quotients(const float (&t)[8]) {
-    const float magic = 12582920.0f;
-    uint32_t ev, od;
-    code_byte<0, true>(ev, t[0], magic);
-    code_byte<0, true>(od, t[1], magic);
-    code_byte<1, false>(ev, t[2], magic);
-    code_byte<1, false>(od, t[3], magic);
-    code_byte<2, false>(ev, t[4], magic);
-    code_byte<2, false>(od, t[5], magic);
-    code_byte<3, false>(ev, t[6], magic);
-    code_byte<3, false>(od, t[7], magic);
-    return ev | (od << 4);
-  }
-
-  // The same word as word4 through code bytes: per code the quotient
-  // y * rcp clamped to [-8, 7] (v_med3; the clamp commutes with the rounding
-  // since -8 and 7 are bf16 values), rounded to bf16 straight into a float32
-  // register by one v_cvt_pk_bf16_f32 whose low half is the conversion of 0.0
-  // (the bf16 value's float32 bits, low half zero), then code_byte: 10 VALU
-  // per pair of codes (the two elements unpacked, two products, two clamps,
-  // two conversions, two code bytes).
-  __device__ static inline uint32_t word_u8(const uint32_t (&p)[4], float rcp) {
-    float t[8];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      // operands are VALU results, never MFMA results
-      asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(t[r]) : "v"(__builtin_amdgcn_fmed3f(lo(p[r]) * rcp, -8.0f, 7.0f)));
-      asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(t[r + 4]) : "v"(__builtin_amdgcn_fmed3f(hi(p[r]) * rcp, -8.0f, 7.0f)));
-    }
-    return word_from_quotients(t);
-  }
-
-  // word_u8 for a token whose largest quotient rounds below 7.5 and whose
-  // smallest rounds to -8.5 or above (every code then lies in -8 .. 7 with
-  // no clamp; the host picks this form from the clip ratio, kNoClampClip):
-  // 8 VALU per pair of codes.
-  __device__ static inline uint32_t word_u8_noclamp(const uint32_t (&p)[4], float rcp) {
-    float t[8];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      // operands are VALU products, never MFMA results
-      asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(t[r]) : "v"(lo(p[r]) * rcp));
-      asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(t[r + 4]) : "v"(hi(p[r]) * rcp));
-    }
-    return word_from_quotients(t);
-  }
-
-  // max |y| of rounded Y pairs as a 16-bit pattern (sign-cleared bf16 bits
-  // order like the values).
-  struct Amax {
-    uint32_t m = 0u;
-  };
-  __device__ static inline void track2(Amax& a, uint32_t p0, uint32_t p1) {
-    a.m = pk_absmax16(pk_absmax16(a.m, p0), p1);
-  }
-  __device__ static inline uint32_t amax_bits(const Amax& a) { return max(a.m & 0xFFFFu, a.m >> 16); }
-};
-
-// LDS transpose read of 16-bit elements (gfx950 ds_read_b64_tr_b16): within
-// each 16-lane group, lane l supplies the address of 4 consecutive elements
-// (8-byte aligned), forming row l of a 16 x 4 matrix A; lane i receives
-// A[i/4][i%4], A[4 + i/4][i%4], A[8 + i/4][i%4], A[12 + i/4][i%4] — that is,
-// A[4e + i/4][i%4] for e = 0..3 (checked on the device).
-typedef short v4s16 __attribute__((ext_vector_type(4)));
-__device__ inline v4s16 lds_tr16(const void* p) {
-  typedef __attribute__((address_space(3))) v4s16* lds_v4s16;
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s16)(__attribute__((address_space(3))) const void*)p);
-}
-// Two 4-element reads as one 8-element MFMA operand (elements 0..3, 4..7).
-template <class V>
-__device__ inline V join_tr16(v4s16 lo, v4s16 hi) {
-  typedef short v8s16 __attribute__((ext_vector_type(8)));
-  const v8s16 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  return __builtin_bit_cast(V, w);
-}
-
 // NV, MV: the token's width and height in memory; N = 32 NP and M = 16 MB are
 // computed, the rest is zero padding (X's padded columns and rows zeroed in
 // registers, R's and L's padded rows and columns zero, padded codes not
 // stored; the padded Y values are 0, which leaves max |Y| unchanged).
-// NV % 8 != 0 (SPLIT; NV even): rows start off 16-byte boundaries, so X is
-// copied in 4-byte pieces, the row's last 8-column chunk is partly padding,
-// and codes are stored in pieces as aligned as the row offset allows: 16-bit
-// (packed) or 4-byte (int8) for NV % 4 == 0, bytes or 16-bit otherwise.
 template <int MB, int NP, int NV = 32 * NP, int MV = 16 * MB>
 struct FqShape {
   static constexpr int M = 16 * MB;
   static constexpr int N = 32 * NP;
   static constexpr int F = MV * NV;
-  static_assert(NV % 2 == 0 && NV > 32 * (NP - 1) && NV <= N, "valid width");
-  static constexpr bool SPLIT = NV % 8 != 0;
+  static_assert(NV % 8 == 0 && NV > 32 * (NP - 1) && NV <= N, "valid width");
   static_assert(MV > 16 * (MB - 1) && MV <= M, "valid height");
   // L's fragments (MB (KS2 + 1) of them, 4 VGPRs each) stay in LDS instead of
   // VGPRs where they would not fit beside R's (2 KS1) and the accumulators.
@@ -645,7 +363,7 @@ struct FqShape {
   static constexpr int WAVES = NP * TPB;
   static constexpr int STAGE_FRAGS = TPB * XFRAGS;
   static constexpr int FRAGS_PER_WAVE = STAGE_FRAGS / WAVES;   // == MB
-  static constexpr int DMA_PER_WAVE = (SPLIT ? 4 : 1) * FRAGS_PER_WAVE;
+  static constexpr int DMA_PER_WAVE = FRAGS_PER_WAVE;
   static constexpr int STAGE_ELEMS = STAGE_FRAGS * 512;
   // One X stage instead of two where two would not fit in LDS beside L's
   // fragments: the next group's copy is then issued once every wave's first
@@ -657,44 +375,6 @@ struct FqShape {
   static_assert(M * M <= STAGE_ELEMS, "L must fit in one X stage while it is staged");
   static_assert(DMA_PER_WAVE < 64, "vmcnt range");
 };
-
-// Wait until at most N vector-memory operations of this wave are outstanding.
-// vmcnt is 6 bits on gfx9 (0..63); the encoding keeps lgkmcnt / expcnt at max.
-template <int N>
-__device__ inline void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt out of range");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-// Codes of one lane's 8 columns (rem of them inside the row, rem > 0) where
-// the row offset in a SPLIT shape allows only partial alignment. Packed: 8
-// nibbles in `word`, at a byte address that is 2-byte aligned when
-// NV % 4 == 0. int8: 8 bytes in lo4 / hi4, at an address 4-byte aligned when
-// NV % 4 == 0, 2-byte aligned otherwise.
-template <int NV>
-__device__ inline void fq_store_packed_split(uint8_t* o, uint32_t word, int rem) {
-  if constexpr (NV % 4 == 0) {
-    reinterpret_cast<uint16_t*>(o)[0] = (uint16_t)word;
-    if (rem >= 8) reinterpret_cast<uint16_t*>(o)[1] = (uint16_t)(word >> 16);
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (2 * k + 2 <= rem) o[k] = (uint8_t)(word >> (8 * k));
-  }
-}
-
-template <int NV>
-__device__ inline void fq_store_int8_split(int8_t* o, uint32_t lo4, uint32_t hi4, int rem) {
-  if constexpr (NV % 4 == 0) {
-    *reinterpret_cast<int32_t*>(o) = (int32_t)lo4;
-    if (rem >= 8) *reinterpret_cast<int32_t*>(o + 4) = (int32_t)hi4;
-  } else {
-    const uint32_t h[4] = {lo4 & 0xFFFFu, lo4 >> 16, hi4 & 0xFFFFu, hi4 >> 16};
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (2 * k + 2 <= rem) reinterpret_cast<uint16_t*>(o)[k] = (uint16_t)h[k];
-  }
-}
 
 // One token group (this wave's token slot and pair) from an X stage in LDS:
 // both products, the per-token scale and the codes.
@@ -714,9 +394,7 @@ __device__ __attribute__((always_inline)) inline void fq_mfma_group(
   constexpr int F = S::F, KS1 = S::KS1, KS2 = S::KS2;
   const int li = lane & 15, lg = lane >> 4;
   // this lane's 8 columns of its pair: stored only inside the valid width
-  // (with SPLIT the last chunk's first rem columns only)
-  const int rem = NV - (32 * q + 8 * lg);
-  const bool col_ok = rem > 0;
+  const bool col_ok = 32 * q + 8 * lg < NV;
 
   // First product, one 16-row block of Z at a time: Z[rb] = X[rb] R[:, pair].
   constexpr int KSL = S::KSL;
@@ -728,14 +406,6 @@ __device__ __attribute__((always_inline)) inline void fq_mfma_group(
     for (int ks = 0; ks < KS1; ++ks) {
       V a = *reinterpret_cast<const V*>(xs + ((rb * KS1 + ks) * 64 + lane) * 8);
       if (NV < S::N && ks == KS1 - 1 && 32 * ks + 8 * lg >= NV) a = V{};   // padded k
-      if (S::SPLIT && ks == KS1 - 1) {                                        // partly padded chunk
-        const int kv = NV - (32 * ks + 8 * lg);
-        if (kv > 0 && kv < 8) {
-#pragma unroll
-          for (int j = 2; j < 8; ++j)
-            if (j >= kv) a[j] = DT::from_f(0.0f);
-        }
-      }
       if (MV < S::M && rb == MB - 1 && 16 * rb + li >= MV) a = V{};        // padded row
       acc0 = Ops::mfma(a, rf[0][ks], acc0);
       acc1 = Ops::mfma(a, rf[1][ks], acc1);
@@ -804,15 +474,7 @@ __device__ __attribute__((always_inline)) inline void fq_mfma_group(
       uint32_t word = 0u - Epi::kJunk;
 #pragma unroll
       for (int r = 0; r < 4; ++r) Epi::accumulate(word, yp[mb][r], rcp, r);
-      if constexpr (S::SPLIT) {
-        // nibble offset t F + m NV + 8 (4q + lg) is even: a byte offset; 16
-        // rows further on is 8 NV bytes further on
-        uint8_t* ob = reinterpret_cast<uint8_t*>(out_codes) + t * (F / 2) + (li * NV + 32 * q + 8 * lg) / 2 +
-                      mb * (8 * NV);
-        if (col_ok && 16 * mb + li < MV) fq_store_packed_split<NV>(ob, word, rem);
-      } else {
-        if (col_ok && 16 * mb + li < MV) orow[(16 * mb + li) * (NV / 8)] = (int32_t)word;
-      }
+      if (col_ok && 16 * mb + li < MV) orow[(16 * mb + li) * (NV / 8)] = (int32_t)word;
     }
     return;
   }
@@ -838,12 +500,7 @@ __device__ __attribute__((always_inline)) inline void fq_mfma_group(
       uint32_t word = 0;
 #pragma unroll
       for (int j = 0; j < 8; ++j) word |= (uint32_t)(code[j] + 8) << (4 * j);
-      if constexpr (S::SPLIT) {
-        uint8_t* ob = reinterpret_cast<uint8_t*>(out_codes) + t * (F / 2) + (m * NV + 32 * q + 8 * lg) / 2;
-        if (col_ok) fq_store_packed_split<NV>(ob, word, rem);
-      } else {
-        if (col_ok) reinterpret_cast<int32_t*>(out_codes)[t * (F / 8) + m * (NV / 8) + 4 * q + lg] = (int32_t)word;
-      }
+      if (col_ok) reinterpret_cast<int32_t*>(out_codes)[t * (F / 8) + m * (NV / 8) + 4 * q + lg] = (int32_t)word;
     } else {
       uint32_t lo4 = 0, hi4 = 0;
 #pragma unroll
@@ -852,12 +509,8 @@ __device__ __attribute__((always_inline)) inline void fq_mfma_group(
         hi4 |= (uint32_t)(code[4 + j] & 0xFF) << (8 * j);
       }
       int8_t* ob = reinterpret_cast<int8_t*>(out_codes) + t * F + m * NV + 32 * q + 8 * lg;
-      if constexpr (S::SPLIT) {
-        if (col_ok) fq_store_int8_split<NV>(ob, lo4, hi4, rem);
-      } else {
-        v2i pair = {(int)lo4, (int)hi4};
-        if (col_ok) *reinterpret_cast<v2i*>(ob) = pair;
-      }
+      v2i pair = {(int)lo4, (int)hi4};
+      if (col_ok) *reinterpret_cast<v2i*>(ob) = pair;
     }
   }
 }
@@ -894,10 +547,7 @@ fq_mfma_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
 
   // LDS-DMA of one token group into a stage. Fragment c of the stage is token
   // slot c / XFRAGS, block (rb, ks); lane l fetches X[16rb + l%16][32ks + 8(l/16) .. +7]
-  // (16 bytes), which the hardware writes to fragment base + 16*l. With SPLIT
-  // each fragment takes four 4-byte copies: copy h, lane l fetches dword l%4 of
-  // fragment lane 16h + l/4, i.e. X[16rb + l/4][32ks + 8h + 2(l%4) .. +1], which
-  // lands at fragment base + 256h + 4l = base + 16(16h + l/4) + 4(l%4).
+  // (16 bytes), which the hardware writes to fragment base + 16*l.
   const int64_t ngroups = (tokens + S::TPB - 1) / S::TPB;
   auto issue = [&](int64_t g, T* stage) {
 #pragma unroll
@@ -907,28 +557,11 @@ fq_mfma_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
       const int rb = fr / KS1, ks = fr % KS1;
       int64_t t = g * S::TPB + ts;
       t = t < tokens ? t : tokens - 1;  // tail slots re-read a valid row; never stored
-      // padded chunks (columns >= NV) re-read the row's last chunk (last dword
-      // with SPLIT); zeroed before use
+      // padded chunks (columns >= NV) re-read the row's last chunk; zeroed before use
       // padded rows (>= MV) re-read the last row; zeroed before use
-      if constexpr (S::SPLIT) {
-        // offsets recomputed at every issue from an opaque lane copy: 4 MB
-        // addresses held across the token loop would not fit in VGPRs
-        int l = lane;
-        asm volatile("" : "+v"(l));
-        const int off = min(16 * rb + (l >> 2), MV - 1) * NV + 2 * (l & 3);
-        const T* xt = x + t * x_ld;
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const T* src = xt + min(off + 32 * ks + 8 * h, min(16 * rb + (l >> 2), MV - 1) * NV + NV - 2);
-          __builtin_amdgcn_global_load_lds((const void*)src,
-                                           (__attribute__((address_space(3))) void*)(stage + c * 512 + h * 128), 4,
-                                           0, 0);
-        }
-      } else {
-        const T* src = x + t * x_ld + min(16 * rb + li, MV - 1) * NV + min(32 * ks + 8 * lg, NV - 8);
-        __builtin_amdgcn_global_load_lds((const void*)src,
-                                         (__attribute__((address_space(3))) void*)(stage + c * 512), 16, 0, 0);
-      }
+      const T* src = x + t * x_ld + min(16 * rb + li, MV - 1) * NV + min(32 * ks + 8 * lg, NV - 8);
+      __builtin_amdgcn_global_load_lds((const void*)src,
+                                       (__attribute__((address_space(3))) void*)(stage + c * 512), 16, 0, 0);
     }
   };
   // Before reading a stage: issue the next group into the other stage (past
@@ -2629,11 +2262,7 @@ static int dispatch_mfma(int M, int N, const void* x, int64_t tokens, int64_t x_
   QO_FQ_CASE(6, 4)   // 96 x 128   (hidden 12288)
   QO_FQ_CASE(4, 3)   // 64 x 96    (hidden 6144)
   QO_FQ_CASE(5, 4)   // 80 x 128   (hidden 10240)
-  QO_FQ_CASE(8, 5)   // 128 x 160  (hidden 20480)
-  QO_FQ_CASE(8, 6)   // 128 x 192  (hidden 24576)
   QO_FQ_CASE(8, 7)   // 128 x 224  (hidden 28672)
-  QO_FQ_CASE(9, 6)   // 144 x 192  (hidden 27648)
-  QO_FQ_CASE(10, 5)  // 160 x 160  (hidden 25600)
   QO_FQ_CASE(8, 8)   // 128 x 256  (hidden 32768; one X stage)
 #undef QO_FQ_CASE
   // widths that are not a multiple of 32: computed zero-padded to 32 NP
@@ -2641,31 +2270,25 @@ static int dispatch_mfma(int M, int N, const void* x, int64_t tokens, int64_t x_
   if (M == 16 * (MB_) && N == (NV_))                                                                     \
     return launch_mfma<DT, MB_, NP_, PACK, NV_>(x, tokens, x_ld, left, right, clip, out_codes, out_scales, \
                                                 stream);
-  QO_FQ_CASE_NV(4, 3, 80)    // 64 x 80   (hidden 5120)
-  QO_FQ_CASE_NV(4, 4, 112)   // 64 x 112  (hidden 7168)
-  QO_FQ_CASE_NV(8, 5, 144)   // 128 x 144 (hidden 18432)
   QO_FQ_CASE_NV(2, 2, 48)    // 32 x 48   (hidden 1536)
   QO_FQ_CASE_NV(4, 3, 88)    // 64 x 88   (hidden 5632)
-  QO_FQ_CASE_NV(5, 4, 112)   // 80 x 112  (hidden 8960)
-  QO_FQ_CASE_NV(8, 5, 148)   // 128 x 148 (hidden 18944; 16-bit code halves)
-  QO_FQ_CASE_NV(8, 6, 172)   // 128 x 172 (hidden 22016; 16-bit code halves)
-  QO_FQ_CASE_NV(4, 7, 214)   // 64 x 214  (hidden 13696; byte code stores)
 #undef QO_FQ_CASE_NV
   // heights that are not a multiple of 16: computed zero-padded to 16 MB
 #define QO_FQ_CASE_MV(MB_, NP_, MV_)                                                                          \
   if (M == (MV_) && N == 32 * (NP_))                                                                          \
     return launch_mfma<DT, MB_, NP_, PACK, 32 * (NP_), MV_>(x, tokens, x_ld, left, right, clip, out_codes,    \
                                                             out_scales, stream);
-  QO_FQ_CASE_MV(4, 2, 56)    // 56 x 64   (hidden 3584)
-  QO_FQ_CASE_MV(6, 4, 86)    // 86 x 128  (hidden 11008)
-  QO_FQ_CASE_MV(7, 4, 108)   // 108 x 128 (hidden 13824)
   QO_FQ_CASE_MV(3, 2, 40)    // 40 x 64   (hidden 2560)
-  QO_FQ_CASE_MV(5, 3, 72)    // 72 x 96   (hidden 6912)
-  QO_FQ_CASE_MV(5, 4, 76)    // 76 x 128  (hidden 9728)
-  // both padded, one X stage
-  if (M == 168 && N == 176)   // 168 x 176 (hidden 29568)
-    return launch_mfma<DT, 11, 6, PACK, 176, 168>(x, tokens, x_ld, left, right, clip, out_codes, out_scales, stream);
 #undef QO_FQ_CASE_MV
+  // Every other shape (scale from max |Y|: clip > 0). The shapes above are those
+  // where fq_mfma_kernel was the faster of the two: whole fragments, which X's
+  // LDS-DMA fills without a pass through registers (4096 tokens bf16: 64 x 96
+  // 24 us against 27, 128 x 224 140 against 151), and small padded ones (40 x 64
+  // 14.2 against 15.5). Padded widths and heights beyond those, and 128 x 160,
+  // 128 x 192, 144 x 192 and 160 x 160, run 5 to 60 % faster on fq_tile_kernel.
+  if (clip > 0.f && clip <= 3.4e38f &&
+      launch_tile<DT>(x, tokens, x_ld, left, right, M, N, clip, PACK ? 1 : 0, out_codes, out_scales, stream))
+    return QO_OK;
   *handled = false;
   return QO_OK;
 }
