@@ -22,9 +22,12 @@
 //                       or LDS, R in VGPRs.
 //  * fq_tile_kernel   — (flatquant_tile.h) fp16 / bf16, every other shape with N
 //                       even up to 256 and M up to 176.
+//  * fq_f32_kernel    — (flatquant_f32.hip) fp32, N up to 256 (even when packing)
+//                       and M up to 128, where X and L fit in LDS: the generic
+//                       kernel's sums, bit for bit, on the float32 matrix cores.
 //  * fq_generic_kernel — any M, N, D in {fp32, fp16, bf16}; VALU fp32 FMA with the
 //                       same rounding points. Used for shapes the MFMA kernels
-//                       do not cover (and for fp32 inputs), X and Z in LDS.
+//                       do not cover, X and Z in LDS.
 //  * fq_generic_big_kernel — the same results where X and Z do not fit in LDS
 //                       (fp32 above 20480 features, other shapes above 40960):
 //                       Y by blocks of 16 columns, computed twice per token.
@@ -43,6 +46,9 @@ namespace qo {
 template <class DT>
 bool launch_tile(const void* x, int64_t tokens, int64_t x_ld, const void* left, const void* right, int M, int N,
                  float clip, int pack, void* out_codes, float* out_scales, hipStream_t stream);
+// fq_f32_kernel (flatquant_f32.hip): the same for float32.
+bool launch_f32(const float* x, int64_t tokens, int64_t x_ld, const float* left, const float* right, int M, int N,
+                float clip, int pack, void* out_codes, float* out_scales, hipStream_t stream);
 
 // ---------------------------------------------------------------------------
 // Generic kernel: one block of BT threads per token (grid-stride over tokens).
@@ -2354,6 +2360,13 @@ static int run_quantize(const void* x, int64_t tokens, int64_t x_ld, const void*
                                        &handled, ra);
       if (handled) return st;
     }
+  } else {
+    // 16-byte loads of X rows and stores of codes; scale from max |Y| (clip > 0)
+    const bool aligned = (uintptr_t)x % 16 == 0 && x_ld % 4 == 0 && (uintptr_t)out_codes % 16 == 0;
+    if (allow_mfma && aligned && clip > 0.f && clip <= 3.4e38f &&
+        launch_f32(reinterpret_cast<const float*>(x), tokens, x_ld, reinterpret_cast<const float*>(left),
+                   reinterpret_cast<const float*>(right), M, N, clip, PACK ? 1 : 0, out_codes, out_scales, stream))
+      return QO_OK;
   }
   return launch_generic<DT, PACK>(x, tokens, x_ld, left, right, M, N, clip, out_codes, out_scales, stream);
 }

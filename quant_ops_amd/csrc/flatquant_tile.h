@@ -63,7 +63,7 @@ __device__ inline void fq_tile_put8(T* at, int col, int pitch, int ncols, v4i v)
 }
 // f(integral_constant<G>) for the largest piece that divides ncols (EVEN: ncols is even).
 template <bool EVEN, class Fn>
-__device__ inline void fq_tile_pieces(int ncols, Fn&& f) {
+__device__ __attribute__((always_inline)) inline void fq_tile_pieces(int ncols, Fn&& f) {
   if ((ncols & 7) == 0) f(std::integral_constant<int, 8>{});
   else if ((ncols & 3) == 0) f(std::integral_constant<int, 4>{});
   else if (EVEN || (ncols & 1) == 0) f(std::integral_constant<int, 2>{});
@@ -210,20 +210,20 @@ fq_tile_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
     const uint32_t e = 8 * (st + i * nts), row = __umulhi(e, d.inv_n), col = e - row * N;
     xat[i] = (row * PX + col) << 8 | col;
   }
-  auto load_x = [&](int64_t t) {
+  auto load_x = [&](int64_t t) __attribute__((always_inline)) {
     const char* src = reinterpret_cast<const char*>(x + (t < tokens ? t : tokens - 1) * x_ld);
 #pragma unroll
     for (int i = 0; i < S::XCH; ++i) xr[i] = *reinterpret_cast<const v4i*>(src + 16u * (uint32_t)min(st + i * nts, nch - 1));
   };
-  auto write_x = [&] {
-    fq_tile_pieces<true>(N, [&](auto gran) {
+  auto write_x = [&]() __attribute__((always_inline)) {
+    fq_tile_pieces<true>(N, [&](auto gran) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < S::XCH; ++i)
         if (st + i * nts < nch)
           fq_tile_put8<decltype(gran)::value>(xs + (xat[i] >> 8), (int)(xat[i] & 255u), PX, N, xr[i]);
     });
   };
-  auto zero_pads = [&] {
+  auto zero_pads = [&]() __attribute__((always_inline)) {
     for (int r = st; r < M; r += nts)
       for (int c = N; c < 32 * KS; c += 2) *reinterpret_cast<int*>(xs + r * PX + c) = 0;
     for (int i = st; i < (16 * d.mb - M) * (PX / 8); i += nts) reinterpret_cast<v4i*>(xs + M * PX)[i] = v4i{0, 0, 0, 0};
@@ -352,7 +352,7 @@ fq_tile_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
       yp[b][1] = Epi::pack_acc(c[2], c[3]);
       if (b % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
-    auto y_at = [&](int b, int r) { return r & 1 ? Epi::hi(yp[b][r >> 1]) : Epi::lo(yp[b][r >> 1]); };
+    auto y_at = [&](int b, int r) __attribute__((always_inline)) { return r & 1 ? Epi::hi(yp[b][r >> 1]) : Epi::lo(yp[b][r >> 1]); };
     // non-negative floats order like their bits; a token of NaNs alone (each wave
     // then reports all ones) takes an infinite scale, as from the empty extremes
     uint32_t top = wave_max_u32(__builtin_bit_cast(uint32_t, amax));
@@ -385,7 +385,7 @@ fq_tile_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
     int lane_at = li * N + 16 * p + 4 * lg;
     asm volatile("" : "+v"(lane_at));   // offsets computed per token instead of held in VGPRs
     // G: 4 where N % 4 == 0 (whole stores), else 2
-    auto codes = [&](auto pk, auto gran, auto&& word) {
+    auto codes = [&](auto pk, auto gran, auto&& word) __attribute__((always_inline)) {
       constexpr bool PK = decltype(pk)::value;
       constexpr int G = decltype(gran)::value;
 #pragma unroll
@@ -407,8 +407,8 @@ fq_tile_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
         }
       }
     };
-    auto nibbles = [&](int b) { return fq_tile_nibbles<DT>(yp[b], rcp); };
-    auto bytes = [&](int b) {
+    auto nibbles = [&](int b) __attribute__((always_inline)) { return fq_tile_nibbles<DT>(yp[b], rcp); };
+    auto bytes = [&](int b) __attribute__((always_inline)) {
       uint32_t w = 0;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -418,7 +418,7 @@ fq_tile_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
       }
       return w;
     };
-    auto slow_nibbles = [&](int b) {
+    auto slow_nibbles = [&](int b) __attribute__((always_inline)) {
       uint32_t w = 0;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -426,7 +426,7 @@ fq_tile_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
       __builtin_amdgcn_sched_barrier(0);
       return w;
     };
-    auto slow_bytes = [&](int b) {
+    auto slow_bytes = [&](int b) __attribute__((always_inline)) {
       uint32_t w = 0;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -456,7 +456,7 @@ fq_tile_kernel(const typename DT::T* __restrict__ x, int64_t tokens, int64_t x_l
     }
     const int64_t gn = g + gridDim.x;
     const bool more = gn < ngroups;
-    auto next_x = [&] {
+    auto next_x = [&]() __attribute__((always_inline)) {
       if (!more) return;
       write_x();
       if (gn + gridDim.x < ngroups) load_x((gn + gridDim.x) * d.tpb + tau);
