@@ -406,6 +406,185 @@ gemm_f6_pp2(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int 
   if (!grp1) bar();
 }
 
+// ---------------------------------------------------------------------------
+// gemm_f6_sm: BM x BN tiles (128 x 128 or 128 x 64) by four waves (2 x 2), two
+// workgroups per CU, for products whose 256-row tiles would leave CUs idle. Each
+// stage is one k-block of the tile's pairs on a three-stage LDS-DMA ring; a
+// wave reads stage t + 1's operands into a second register set while it
+// multiplies stage t, so a stage costs one barrier: it says that stage t + 1
+// has landed and that every wave holds stage t in registers, which frees its
+// slot for the copies of stage t + 3.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, class OT>
+__global__ void __launch_bounds__(256, 2)
+gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int pr_a, int pr_b, int nk,
+           const void* __restrict__ sa, int sad, const void* __restrict__ sb, int sbd,
+           typename OT::T* __restrict__ out, int64_t ldc, const typename OT::T* __restrict__ bias, int M, int N,
+           int tiles_m) {
+  constexpr int W = 4, STAGES = 3;
+  using S = F6Stage<BM, BN>;
+  using T = typename OT::T;
+  constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16, QA = FM / 2, QB = FN / 2;
+  constexpr int PER = (S::DMA + W - 1) / W, TA = S::A_DMA / W;
+  static_assert(sizeof(T) == 2, "16-bit outputs (staged epilogue)");
+  static_assert(S::A_DMA % W == 0 && FM % 2 == 0 && FN % 2 == 0 && BM <= 128 && BN <= 128, "tile");
+  constexpr int C_PITCH = BN * 2 + 16;
+  __shared__ __align__(16) unsigned char ring[STAGES * S::BYTES];
+  static_assert(PER * (STAGES - 1) < 64, "vmcnt range");
+  static_assert(BM * C_PITCH <= STAGES * S::BYTES, "staged output");
+  __shared__ __align__(16) float s_sa[BM];
+  __shared__ __align__(16) float s_sb[BN];
+  __shared__ __align__(16) float s_bias[BN];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int li = lane & 15, lg = lane >> 4;
+
+  // Each XCD (workgroup j runs on XCD j % 8) a contiguous run of tiles, in
+  // groups of up to 8 row tiles x every column tile, row tiles first: a column
+  // tile of B is read by its row tiles from one L2.
+  const int nblk = gridDim.x, xcd = blockIdx.x & 7;
+  const int pid = xcd * (nblk >> 3) + min(xcd, nblk & 7) + (int)(blockIdx.x >> 3);
+  constexpr int GM = 8;
+  const int tiles_n = (N + BN - 1) / BN;
+  const int g = pid / (GM * tiles_n), w = pid % (GM * tiles_n);
+  const int gm = min(GM, tiles_m - g * GM);
+  const int tm = g * GM + w % gm, tn = w / gm;
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  // copies as in gemm_f6_pp2: copy t of this wave is stage instruction wave + 4 t
+  const int64_t prs = (int64_t)nk * kF6Pair;   // bytes per pair row
+  const uint8_t* const a_base = a6 + (int64_t)(m0 >> 5) * prs;
+  const uint8_t* const b_base = b6 + (int64_t)(n0 >> 5) * prs;
+  uint32_t dst[PER], voff[PER];
+#pragma unroll
+  for (int t = 0; t < PER; ++t) {
+    int i = wave + W * t;
+    i = i < S::DMA ? i : S::DMA - 1;
+    const int o = 1024 * i + 16 * lane;
+    if (t < TA) {
+      const int f = min(o / kF6Pair, pr_a - 1 - (m0 >> 5));
+      voff[t] = (uint32_t)(f * prs + o % kF6Pair);
+    } else {
+      const int ob = o - S::A_BYTES;
+      const int f = min(ob / kF6Pair, pr_b - 1 - (n0 >> 5));
+      voff[t] = (uint32_t)(f * prs + ob % kF6Pair);
+    }
+    dst[t] = __builtin_amdgcn_readfirstlane((uint32_t)(1024 * i));
+  }
+  const uint32_t ring0 = lds_addr(ring);
+  auto issue = [&](int ks, int slot) __attribute__((always_inline)) {
+    const uint32_t base = ring0 + slot * S::BYTES;
+    const uint8_t* ab = a_base + (int64_t)ks * kF6Pair;
+    const uint8_t* bb = b_base + (int64_t)ks * kF6Pair;
+#pragma unroll
+    for (int t = 0; t < PER; ++t) dma16_s(voff[t], t < TA ? ab : bb, base + dst[t]);
+  };
+
+  v16i ap[2][QA], bp[2][QB];
+  auto pair_at = [](const unsigned char* p) __attribute__((always_inline)) -> v16i {
+    const v4i x0 = *reinterpret_cast<const v4i*>(p), x1 = *reinterpret_cast<const v4i*>(p + 1024),
+              x2 = *reinterpret_cast<const v4i*>(p + 2048);
+    return v16i{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3], x2[0], x2[1], x2[2], x2[3], 0, 0, 0, 0};
+  };
+  auto load_regs = [&](auto setc, int slot) __attribute__((always_inline)) {
+    constexpr int H = decltype(setc)::value;
+    const unsigned char* base = ring + slot * S::BYTES + 16 * lane;
+#pragma unroll
+    for (int q = 0; q < QA; ++q) ap[H][q] = pair_at(base + (wm * QA + q) * kF6Pair);
+#pragma unroll
+    for (int q = 0; q < QB; ++q) bp[H][q] = pair_at(base + S::A_BYTES + (wn * QB + q) * kF6Pair);
+  };
+  auto half = [](const v16i& v, int odd) __attribute__((always_inline)) -> v8i {
+    return odd ? __builtin_shufflevector(v, v, 6, 7, 8, 9, 10, 11, 12, 13)
+               : __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+
+  v4f acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  // The tile's scales and bias as raw bits, requested before the copies and
+  // converted after the last stage.
+  auto raw = [](const void* p, int dtype, int64_t i) __attribute__((always_inline)) -> uint32_t {
+    return dtype == QO_DTYPE_F32 ? reinterpret_cast<const uint32_t*>(p)[i] : reinterpret_cast<const uint16_t*>(p)[i];
+  };
+  uint32_t rs = 0, rbias = 0;
+  if (tid < 128) {
+    rs = raw(sa, sad, min(m0 + tid, M - 1));
+  } else {
+    const int jn = min(n0 + tid - 128, N - 1);
+    rs = raw(sb, sbd, jn);
+    if (bias) rbias = raw(bias, QO_DTYPE_F16, jn);
+  }
+
+#pragma unroll
+  for (int t = 0; t < STAGES; ++t)
+    if (t < nk) issue(t, t);
+  gemm_wait_groups<PER, STAGES - 1>(nk - 1);
+  raw_barrier();
+  load_regs(std::integral_constant<int, 0>{}, 0);
+
+  int slot = 0;   // of stage t
+  auto stage = [&](int t, auto setc) __attribute__((always_inline)) {
+    constexpr int H = decltype(setc)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    gemm_wait_groups<PER, STAGES - 2>(nk - 2 - t);   // stage t + 1 has landed (the later ones may be in flight)
+    __builtin_amdgcn_s_waitcnt(0xC07F);     // lgkmcnt(0): stage t is in this wave's registers
+    raw_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const int next = slot == STAGES - 1 ? 0 : slot + 1;
+    if (t + STAGES < nk) issue(t + STAGES, slot);
+    if (t + 1 < nk) load_regs(std::integral_constant<int, 1 - H>{}, next);
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+            half(bp[H][j >> 1], j & 1), half(ap[H][i >> 1], i & 1), acc[i][j], 2, 2, 0, 130, 0, 130);
+    slot = next;
+  };
+  for (int t = 0; t < nk; t += 2) {
+    stage(t, std::integral_constant<int, 0>{});
+    if (t + 1 < nk) stage(t + 1, std::integral_constant<int, 1>{});
+  }
+
+  // acc[i][j][r] is row wm * WM + 16 i + li, column wn * WN + 16 j + 4 lg + r;
+  // its value is the integer sum itself (exact in float32).
+  asm volatile("" : "+v"(rs), "+v"(rbias));
+  if (tid < 128) {
+    if (tid < BM) s_sa[tid] = scale_from_bits(rs, sad);
+  } else if (tid - 128 < BN) {
+    s_sb[tid - 128] = scale_from_bits(rs, sbd);
+    s_bias[tid - 128] = (float)__builtin_bit_cast(T, (uint16_t)rbias);
+  }
+  __syncthreads();   // also: no wave reads the ring any more
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int row = wm * WM + 16 * i + li;
+    const float sav = s_sa[row];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int c = wn * WN + 16 * j + 4 * lg;
+      const v4f sbv = *reinterpret_cast<const v4f*>(s_sb + c);
+      T v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = OT::cvt((acc[i][j][r] * sav) * sbv[r]);
+      if (bias) {
+        const v4f bb = *reinterpret_cast<const v4f*>(s_bias + c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = OT::cvt((float)v[r] + bb[r]);
+      }
+      *reinterpret_cast<v2i*>(ring + row * C_PITCH + 2 * c) =
+          v2i{(int)(out_bits<OT>(v[0]) | out_bits<OT>(v[1]) << 16), (int)(out_bits<OT>(v[2]) | out_bits<OT>(v[3]) << 16)};
+    }
+  }
+  lds_barrier();
+  copy_out_c<BM, BN, 256, OT, true>(ring, C_PITCH, out, ldc, M, N, m0, n0, tid);
+}
+
 // Job for operand rows [R, K] given by (src, strides): row r's word p at
 // src[r * s_r + p * s_p], with s_p == 1 (row-major) or s_r == 1.
 F6Job f6_job(const int32_t* src, int64_t s_r, int64_t s_p, int64_t R, int64_t K, uint8_t* dst) {
@@ -435,12 +614,31 @@ int64_t f6_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 }
 
 namespace {
-// column tile: 224 or 256, whichever leaves fewer idle CU slots over the rounds
-bool f6_wide(int64_t M, int64_t N) {
-  const int cus = device_cu_count();
-  const int64_t tiles_m = (M + 255) / 256;
-  const int64_t t224 = tiles_m * ((N + 223) / 224), t256 = tiles_m * ((N + 255) / 256);
-  return ((t256 + cus - 1) / cus) * 256 < ((t224 + cus - 1) / cus) * 224;
+// The output tile of an M x N x K product, by an estimate of its time in ns: k-blocks
+// times the time of a round's stages, plus what a round takes besides them. A
+// stage is bound by the CU's LDS traffic (its operand reads at about 128 bytes
+// per clock, the copies from L2 at 64), so a larger tile costs less per product
+// but leaves more CUs idle. Per stage, measured at 4096 columns x 14336: 256-row
+// tiles 740 (850 with every CU busy, 256 columns wide), 128 x 128 430 for one
+// workgroup on a CU and 700 for two, 128 x 64 345 and 480; per round 8 us and 4 us.
+// With 256-row tiles alone M = 512 took 83.7 us there (38 tiles on 256 CUs), on
+// 128 x 64 it takes 40 us; 512 x 14336 x 4096 33 -> 25 us on 128 x 128; 2048 x
+// 4096 x 4096 34 -> 25 us; 2048 x 14336 x 4096 keeps 256 x 224 (87 us against 94).
+enum F6Tile { kF6Tile224, kF6Tile256, kF6Tile128, kF6Tile64 };
+F6Tile f6_tile(int64_t M, int64_t N, int64_t K) {
+  const int64_t cus = device_cu_count(), nk = (K + 127) / 128;
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  auto wide = [&](int64_t t, int64_t stage) { return (t + cus - 1) / cus * (nk * stage + 8000); };
+  auto pair = [&](int64_t t, int64_t one, int64_t two) {   // rounds of two workgroups per CU
+    const int64_t full = t / (2 * cus), rest = t % (2 * cus);
+    return full * (nk * two + 4000) + (rest == 0 ? 0 : nk * (rest <= cus ? one : two) + 4000);
+  };
+  const int64_t est[4] = {wide(tiles(256, 224), 745), wide(tiles(256, 256), 850), pair(tiles(128, 128), 430, 700),
+                          pair(tiles(128, 64), 345, 480)};
+  int best = 0;
+  for (int i = 1; i < 4; ++i)
+    if (est[i] < est[best]) best = i;
+  return (F6Tile)best;
 }
 }  // namespace
 
@@ -471,17 +669,19 @@ void f6_run(const void* sa, int sad, const void* sb, int sbd, typename OT::T* ou
 template <class OT>
 void f6_run2(const void* a6v, const void* b6v, const void* sa, int sad, const void* sb, int sbd, typename OT::T* out,
              int64_t ldc, const typename OT::T* bias, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
-  constexpr int BM = 256;
   const uint8_t* a6 = static_cast<const uint8_t*>(a6v);
   const uint8_t* b6 = static_cast<const uint8_t*>(b6v);
-  const bool wide = f6_wide(M, N);
-  const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + (wide ? 255 : 223)) / (wide ? 256 : 224));
-  auto go = [&](auto kernel) {
-    launch(kernel, dim3(tiles_m * tiles_n), dim3(512), 0, stream, a6, b6, (int)((M + 31) / 32), (int)((N + 31) / 32),
-           (int)((K + 127) / 128), sa, sad, sb, sbd, out, ldc, bias, (int)M, (int)N, tiles_m);
+  auto go = [&](auto kernel, int bm, int bn, int threads) {
+    const int tiles_m = (int)((M + bm - 1) / bm), tiles_n = (int)((N + bn - 1) / bn);
+    launch(kernel, dim3(tiles_m * tiles_n), dim3(threads), 0, stream, a6, b6, (int)((M + 31) / 32),
+           (int)((N + 31) / 32), (int)((K + 127) / 128), sa, sad, sb, sbd, out, ldc, bias, (int)M, (int)N, tiles_m);
   };
-  if (wide) go(gemm_f6_pp2<BM, 256, OT>);
-  else go(gemm_f6_pp2<BM, 224, OT>);
+  switch (f6_tile(M, N, K)) {
+    case kF6Tile224: go(gemm_f6_pp2<256, 224, OT>, 256, 224, 512); break;
+    case kF6Tile256: go(gemm_f6_pp2<256, 256, OT>, 256, 256, 512); break;
+    case kF6Tile128: go(gemm_f6_sm<128, 128, OT>, 128, 128, 256); break;
+    case kF6Tile64: go(gemm_f6_sm<128, 64, OT>, 128, 64, 256); break;
+  }
 }
 
 template <class OT>

@@ -1,0 +1,42 @@
+"""The FP6 GEMM's output tiles at ragged edges, each against the integer route,
+whose sums are exact: outputs are equal bit for bit. The host picks the tile from
+the sizes; which one it is for each case here is in its comment."""
+import pytest
+import torch
+
+from quant_ops_amd import capi
+from quant_ops_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    (257, 100, 8),          # 128 x 64, one k-block
+    (300, 333, 136),        # 128 x 64, two
+    (513, 1000, 1000),      # 128 x 64, more k-blocks than the ring has stages
+    (333, 11001, 392),      # 128 x 128, odd N
+    (700, 5003, 1160),      # 128 x 128
+    (1025, 14329, 776),     # 128 x 128, several rounds of workgroups
+    (1000, 14001, 640),     # 256 x 224, odd N
+    (4090, 4099, 2056),     # 256 x 224
+    (4001, 4090, 1032),     # 256 x 256
+]
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", CASES)
+def test_f6_tile_equals_integer_route(gpu, m, n, k, out_dtype, bias):
+    print(f"[gpu-f6-tiles] {m}x{n}x{k} {out_dtype} bias={bias}", flush=True)
+    case = wl.gemm_case(m, n, k, seed=m + k, b_transposed_view=(m + n) % 2 == 0, out_dtype=out_dtype)
+    a, b = case.a.to(gpu), case.b.to(gpu)
+    sa, sb = case.scale_a.to(gpu).float(), case.scale_b.to(gpu)
+    bv = wl.uniform(n, -1.0, 1.0, 7, out_dtype).to(gpu) if bias else None
+    ws = torch.empty(capi.f6_workspace_bytes(m, n, k), dtype=torch.uint8, device=gpu)
+    capi.f6_prepare(ws, m, n, k, a=a, b=b)
+    wide = torch.full((m, n + 3), 7.0, dtype=out_dtype, device=gpu)   # rows at a stride above their length
+    out = wide[:, :n]
+    capi.f6_run(ws, m, n, k, sa, sb, out_dtype=out_dtype, out=out, bias=bv)
+    with capi.kernel_routing("GEMM_NO_F6"):
+        ref = capi.int4_gemm(a, b, sa, sb, out_dtype=out_dtype, bias=bv)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref) and bool((wide[:, n:] == 7.0).all())
