@@ -178,8 +178,9 @@ int qo_int4_gemm_ws(const int32_t* a, int64_t lda,
 
 /*
  * Workspace bytes qo_int4_gemm_ws uses for an M x N x K product with outputs
- * of out_dtype: 0 when the shape does not take the FP6 route (M <= 256, float32
- * outputs, K > 65536, or QO_ROUTE_GEMM_NO_F6 or QO_ROUTE_GEMM_GENERIC set), else
+ * of out_dtype: 0 when the shape does not take the FP6 route (M <= 256 or float32
+ * outputs where N % 4 == 0 and K % 128 == 0, K > 65536, or QO_ROUTE_GEMM_NO_F6 or
+ * QO_ROUTE_GEMM_GENERIC set), else
  * qo_int4_gemm_f6_workspace_bytes(M, N, K): 0.75 (M + N) K bytes plus padding
  * (M and N up to multiples of 32, K up to a multiple of 128).
  */

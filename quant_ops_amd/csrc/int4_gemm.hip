@@ -889,6 +889,8 @@ struct SkinnyEpilogue {
     }
   }
 
+  // ANY: rows of the output at any alignment, else 4-element aligned
+  template <bool ANY = false>
   __device__ void store(const v4i& sum, int sad, int sbd, const T* bias, T* out, int64_t ldc, int m, int nc,
                         int N) const {
     const float sam = scale_from_bits(sa_bits, sad);
@@ -899,7 +901,7 @@ struct SkinnyEpilogue {
       v[r] = bias ? OT::cvt((float)o + (float)bias_v[r]) : o;
     }
     T* o = out + (int64_t)m * ldc + nc;
-    if (nc + 3 < N) {
+    if (nc + 3 < N && (!ANY || (((uintptr_t)out | (uint64_t)ldc * sizeof(T)) % (4 * sizeof(T))) == 0)) {   // nc % 4 == 0
       if constexpr (sizeof(T) == 2) {
         typedef short v4s __attribute__((ext_vector_type(4)));
         v4s pk;
@@ -1060,7 +1062,10 @@ struct SkinnyNkCfg {
   static_assert(!PAIR || (PAIR_OK && RING * BUF <= 80 * 1024), "two workgroups per CU");
 };
 
-template <int MT, bool PAIR, bool KN, class OT>
+// RAGGED: K % 128 != 0 (whole 16-byte pieces, K % 32 == 0) or output rows not
+// 4-element aligned; a form of its own because the same kernel with both cases
+// inside took 4 % longer on every other call.
+template <int MT, bool PAIR, bool KN, class OT, bool RAGGED = false>
 __global__ void __launch_bounds__(512)
 gemm_i4_skinny_nk(const int32_t* __restrict__ a, int64_t lda, const int32_t* __restrict__ b, int64_t ldb,
                   const void* __restrict__ sa, int sad, const void* __restrict__ sb, int sbd,
@@ -1077,7 +1082,9 @@ gemm_i4_skinny_nk(const int32_t* __restrict__ a, int64_t lda, const int32_t* __r
   const int nblk = gridDim.x;
   const int cblk = KN && nblk % 8 == 0 ? (blockIdx.x & 7) * (nblk >> 3) + (blockIdx.x >> 3) : blockIdx.x;
   const int n0 = cblk * 16;
-  const int nk = K >> 7;                        // stages
+  const int nk = RAGGED ? (K + 127) >> 7 : K >> 7;   // stages
+  // the last stage's lane groups past the row's end multiply B words of code 8 (q = 0)
+  const int tail = RAGGED ? (K & 127) >> 5 : 0;      // valid lane groups of the last stage (0: all four)
   const int rowbytes = K >> 1;                  // bytes of a packed row
   const int nch = (rowbytes + C::CB - 1) / C::CB;
 
@@ -1152,6 +1159,10 @@ gemm_i4_skinny_nk(const int32_t* __restrict__ a, int64_t lda, const int32_t* __r
       } else {
         bw = *reinterpret_cast<const v4i*>(base + li * C::CB + 16 * slot);
       }
+      if (RAGGED && tail != 0 && c * C::SPC + ls == nk - 1) {
+        const int q0 = (int)0x88888888u;
+        bw = lg < tail ? bw : v4i{q0, q0, q0, q0};
+      }
       v4i aw[MT];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
@@ -1210,7 +1221,7 @@ gemm_i4_skinny_nk(const int32_t* __restrict__ a, int64_t lda, const int32_t* __r
   const int m = 16 * mt + li;
   const int nc = n0 + 4 * lg;
   if (m >= M || nc >= N) return;
-  epi.store(sum, sad, sbd, bias, out, ldc, m, nc, N);
+  epi.template store<RAGGED>(sum, sad, sbd, bias, out, ldc, m, nc, N);
 }
 
 // ---------------------------------------------------------------------------
@@ -1318,13 +1329,20 @@ static void launch_skinny(const int32_t* a, int64_t lda, const int32_t* b, int64
   // The LDS-DMA kernel for both layouts; [K/8, N] needs whole 4-column groups
   // and 32-bit byte offsets over B, else the register-streaming kernel.
   const bool kn_dma = !b_nk && skinny_kn_dma_ok(N, K, ldb);
+  const bool ragged = K % 128 != 0 || (uintptr_t)out % (4 * sizeof(T)) != 0 || ldc % 4 != 0;
   auto go = [&](auto mt, auto nk_layout) {
     constexpr int MT = decltype(mt)::value;
     constexpr bool NK = decltype(nk_layout)::value;
     using Cfg = SkinnyNkCfg<MT, false>;
     const int64_t cb = Cfg::CB;
     const bool pair = (K / 2 + cb - 1) / cb <= 2 || (N + 15) / 16 > device_cu_count();
-    if (NK || kn_dma) {
+    if ((NK || kn_dma) && ragged) {
+      if constexpr (MT <= 4)
+        launch((gemm_i4_skinny_nk<MT, false, !NK, OT, true>), grid, dim3(512), 0, stream, a, lda, b, ldb, sa, sad, sb,
+               sbd, reinterpret_cast<T*>(out), ldc, reinterpret_cast<const T*>(bias), M, N, K);
+      else if (g_launch_error == hipSuccess)
+        g_launch_error = hipErrorInvalidConfiguration;   // the host sends ragged shapes here up to 64 rows
+    } else if (NK || kn_dma) {
       bool launched = false;
       if constexpr (Cfg::PAIR_OK) {
         if (pair) {
@@ -1360,12 +1378,24 @@ static void launch_skinny(const int32_t* a, int64_t lda, const int32_t* b, int64
   else by_layout(std::integral_constant<int, 8>{});
 }
 
-// Shapes that take the FP6 route when the caller gives a workspace: the
-// tiled shapes (more than 256 rows; fewer take the small-M kernels), 16-bit
-// outputs, B with one unit stride, K within the exact float32 range.
+// Shapes whose rows the integer tiled kernels cannot take (stores of 4 columns,
+// stages of 128 k): without a workspace they run on the register-staged or the
+// generic kernel, a few per cent of the rate.
+static bool ragged(int64_t N, int64_t K) { return N % 4 != 0 || K % 128 != 0; }
+
+// Shapes that take the FP6 route when the caller gives a workspace: the tiled
+// shapes (more than 256 rows; fewer take the small-M kernels) with 16-bit
+// outputs, and ragged ones of any M and output type; B with one unit stride, K
+// within the exact float32 range. Measured against the kernels these ran on
+// before (N x K = 1631 x 8064, bf16 out): 200 rows 641 -> 33 us (W.t()), 16 rows
+// of [K/8, N] 341 -> 30 us; 200 x 1632 x 8128 181 -> 33 us; 315 x 5478 x 11008,
+// float32 out, 4983 -> 60 us. Up to 64 rows of W.t() stay on the small-M kernel
+// (16 x 1631 x 8064 164 -> 6.6 us).
 static bool f6_route(int64_t M, int64_t N, int64_t K, int out_dtype, int64_t bsp, int64_t bsn) {
-  return (out_dtype == QO_DTYPE_F16 || out_dtype == QO_DTYPE_BF16) && M > 256 && N >= 1 && K >= 8 && K <= 65536 &&
-         M <= INT32_MAX / 2 && N <= INT32_MAX / 2 && (bsp == 1 || bsn == 1) && !route_off(QO_ROUTE_GEMM_NO_F6);
+  const bool f32 = out_dtype == QO_DTYPE_F32;
+  return (f32 || out_dtype == QO_DTYPE_F16 || out_dtype == QO_DTYPE_BF16) && ((M > 256 && !f32) || ragged(N, K)) &&
+         M >= 1 && N >= 1 && K >= 8 && K <= 65536 && M <= INT32_MAX / 2 && N <= INT32_MAX / 2 &&
+         (bsp == 1 || bsn == 1) && !route_off(QO_ROUTE_GEMM_NO_F6);
 }
 
 template <class OT>
@@ -1373,31 +1403,32 @@ static void dispatch(const int32_t* a, int64_t lda, const int32_t* b, int64_t bs
                      int sad, const void* sb, int sbd, void* out, int64_t ldc, const void* bias, int64_t M, int64_t N, int64_t K,
                      hipStream_t stream, bool allow_fast, void* workspace, int64_t ws_bytes) {
   using T = typename OT::T;
-  if constexpr (sizeof(T) == 2) {
-    if (allow_fast && workspace && (uintptr_t)workspace % 256 == 0 &&
-        f6_route(M, N, K, std::is_same_v<OT, OutF16> ? QO_DTYPE_F16 : QO_DTYPE_BF16, bsp, bsn) &&
-        ws_bytes >= f6_workspace_bytes(M, N, K)) {
-      f6_gemm_launch<OT>(a, lda, b, bsp, bsn, sa, sad, sb, sbd, static_cast<T*>(out), ldc,
-                         static_cast<const T*>(bias), M, N, K, workspace, stream);
-      return;
-    }
-  }
+  constexpr int kOut = std::is_same_v<OT, OutF16> ? QO_DTYPE_F16 : std::is_same_v<OT, OutBF16> ? QO_DTYPE_BF16 : QO_DTYPE_F32;
+  const bool f6 = allow_fast && workspace && (uintptr_t)workspace % 256 == 0 && f6_route(M, N, K, kOut, bsp, bsn) &&
+                  ws_bytes >= f6_workspace_bytes(M, N, K);
   const bool b_nk = (bsp == 1);
   const bool b_kn = (bsn == 1) && !b_nk;
   const int64_t ldb = b_nk ? bsn : bsp;
   // 32-bit in-tile byte offsets of the pipelined kernels: 256 rows of A or B
   const bool fits = M <= INT32_MAX / 2 && N <= INT32_MAX / 2 && K <= 65536 && lda < (1 << 21) &&
                     ldb < (1 << 21);
-  const bool aligned = ((uintptr_t)a % 16 == 0) && (lda % 4 == 0) && ((uintptr_t)b % 16 == 0) && (ldb % 4 == 0) &&
-                       ((uintptr_t)out % (4 * sizeof(T)) == 0) && (ldc % 4 == 0);
+  const bool aligned_in = ((uintptr_t)a % 16 == 0) && (lda % 4 == 0) && ((uintptr_t)b % 16 == 0) && (ldb % 4 == 0);
+  const bool aligned = aligned_in && ((uintptr_t)out % (4 * sizeof(T)) == 0) && (ldc % 4 == 0);
+  const bool dma_layout = b_nk || skinny_kn_dma_ok(N, K, ldb);
+  // decode shapes: the skinny kernel (columns x K-slices, B streamed once); the
+  // LDS-DMA form also takes rows of whole 16-byte pieces that end inside a stage
+  if (allow_fast && fits && aligned_in && (b_nk || b_kn) && M <= 64 && K > 0 && gemm_allow_skinny() &&
+      (K % 128 == 0 || (K % 32 == 0 && dma_layout)) && (b_nk || dma_layout || aligned)) {
+    launch_skinny<OT>(a, lda, b, ldb, b_nk, sa, sad, sb, sbd, out, ldc, bias, (int)M, (int)N, (int)K, stream);
+    return;
+  }
+  if (f6) {
+    f6_gemm_launch<OT>(a, lda, b, bsp, bsn, sa, sad, sb, sbd, static_cast<T*>(out), ldc, static_cast<const T*>(bias),
+                       M, N, K, workspace, stream);
+    return;
+  }
   if (allow_fast && fits && aligned && (b_nk || b_kn)) {
     const int m = (int)M, n = (int)N, k = (int)K;
-    // decode shapes: the skinny kernel (columns x K-slices, B streamed once)
-    const bool dma_layout = b_nk || skinny_kn_dma_ok(n, k, ldb);
-    if (m <= 64 && k % 128 == 0 && k > 0 && gemm_allow_skinny()) {
-      launch_skinny<OT>(a, lda, b, ldb, b_nk, sa, sad, sb, sbd, out, ldc, bias, m, n, k, stream);
-      return;
-    }
     // Up to 256 rows over few columns (the tiled grid would fill at most 1/8
     // of the CUs, each tile streaming all of K): one skinny launch per 128
     // rows. Measured at N x K = 4096 x 14336, M = 128 / 200 / 256 / 512:

@@ -426,7 +426,7 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
   using T = typename OT::T;
   constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16, QA = FM / 2, QB = FN / 2;
   constexpr int PER = (S::DMA + W - 1) / W, TA = S::A_DMA / W;
-  static_assert(sizeof(T) == 2, "16-bit outputs (staged epilogue)");
+  constexpr bool kF32 = sizeof(T) == 4;   // float32 outputs are stored from registers, 16-bit ones through LDS
   static_assert(S::A_DMA % W == 0 && FM % 2 == 0 && FN % 2 == 0 && BM <= 128 && BN <= 128, "tile");
   constexpr int C_PITCH = BN * 2 + 16;
   __shared__ __align__(16) unsigned char ring[STAGES * S::BYTES];
@@ -517,7 +517,7 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
   } else {
     const int jn = min(n0 + tid - 128, N - 1);
     rs = raw(sb, sbd, jn);
-    if (bias) rbias = raw(bias, QO_DTYPE_F16, jn);
+    if (bias) rbias = raw(bias, kF32 ? QO_DTYPE_F32 : QO_DTYPE_F16, jn);
   }
 
 #pragma unroll
@@ -558,9 +558,11 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
     if (tid < BM) s_sa[tid] = scale_from_bits(rs, sad);
   } else if (tid - 128 < BN) {
     s_sb[tid - 128] = scale_from_bits(rs, sbd);
-    s_bias[tid - 128] = (float)__builtin_bit_cast(T, (uint16_t)rbias);
+    if constexpr (kF32) s_bias[tid - 128] = __builtin_bit_cast(float, rbias);
+    else s_bias[tid - 128] = (float)__builtin_bit_cast(T, (uint16_t)rbias);
   }
   __syncthreads();   // also: no wave reads the ring any more
+  const bool vec = kF32 && (uintptr_t)out % 16 == 0 && ldc % 4 == 0;
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
     const int row = wm * WM + 16 * i + li;
@@ -577,12 +579,27 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = OT::cvt((float)v[r] + bb[r]);
       }
-      *reinterpret_cast<v2i*>(ring + row * C_PITCH + 2 * c) =
-          v2i{(int)(out_bits<OT>(v[0]) | out_bits<OT>(v[1]) << 16), (int)(out_bits<OT>(v[2]) | out_bits<OT>(v[3]) << 16)};
+      if constexpr (kF32) {
+        const int m = m0 + row, n = n0 + c;
+        if (m >= M) continue;
+        T* const o = out + (int64_t)m * ldc + n;
+        if (vec && n + 3 < N) {
+          *reinterpret_cast<v4f*>(o) = v4f{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < N) o[r] = v[r];
+        }
+      } else {
+        *reinterpret_cast<v2i*>(ring + row * C_PITCH + 2 * c) =
+            v2i{(int)(out_bits<OT>(v[0]) | out_bits<OT>(v[1]) << 16), (int)(out_bits<OT>(v[2]) | out_bits<OT>(v[3]) << 16)};
+      }
     }
   }
-  lds_barrier();
-  copy_out_c<BM, BN, 256, OT, true>(ring, C_PITCH, out, ldc, M, N, m0, n0, tid);
+  if constexpr (!kF32) {
+    lds_barrier();
+    copy_out_c<BM, BN, 256, OT, true>(ring, C_PITCH, out, ldc, M, N, m0, n0, tid);
+  }
 }
 
 // Job for operand rows [R, K] given by (src, strides): row r's word p at
@@ -625,7 +642,7 @@ namespace {
 // 128 x 64 it takes 40 us; 512 x 14336 x 4096 33 -> 25 us on 128 x 128; 2048 x
 // 4096 x 4096 34 -> 25 us; 2048 x 14336 x 4096 keeps 256 x 224 (87 us against 94).
 enum F6Tile { kF6Tile224, kF6Tile256, kF6Tile128, kF6Tile64 };
-F6Tile f6_tile(int64_t M, int64_t N, int64_t K) {
+F6Tile f6_tile(int64_t M, int64_t N, int64_t K, bool f32) {
   const int64_t cus = device_cu_count(), nk = (K + 127) / 128;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   auto wide = [&](int64_t t, int64_t stage) { return (t + cus - 1) / cus * (nk * stage + 8000); };
@@ -635,8 +652,8 @@ F6Tile f6_tile(int64_t M, int64_t N, int64_t K) {
   };
   const int64_t est[4] = {wide(tiles(256, 224), 745), wide(tiles(256, 256), 850), pair(tiles(128, 128), 430, 700),
                           pair(tiles(128, 64), 345, 480)};
-  int best = 0;
-  for (int i = 1; i < 4; ++i)
+  int best = f32 ? 2 : 0;   // the 256-row kernel stages 16-bit values
+  for (int i = best + 1; i < 4; ++i)
     if (est[i] < est[best]) best = i;
   return (F6Tile)best;
 }
@@ -676,9 +693,14 @@ void f6_run2(const void* a6v, const void* b6v, const void* sa, int sad, const vo
     launch(kernel, dim3(tiles_m * tiles_n), dim3(threads), 0, stream, a6, b6, (int)((M + 31) / 32),
            (int)((N + 31) / 32), (int)((K + 127) / 128), sa, sad, sb, sbd, out, ldc, bias, (int)M, (int)N, tiles_m);
   };
-  switch (f6_tile(M, N, K)) {
-    case kF6Tile224: go(gemm_f6_pp2<256, 224, OT>, 256, 224, 512); break;
-    case kF6Tile256: go(gemm_f6_pp2<256, 256, OT>, 256, 256, 512); break;
+  constexpr bool kF32 = std::is_same_v<OT, OutF32>;
+  switch (f6_tile(M, N, K, kF32)) {
+    case kF6Tile224:
+      if constexpr (!kF32) go(gemm_f6_pp2<256, 224, OT>, 256, 224, 512);
+      break;
+    case kF6Tile256:
+      if constexpr (!kF32) go(gemm_f6_pp2<256, 256, OT>, 256, 256, 512);
+      break;
     case kF6Tile128: go(gemm_f6_sm<128, 128, OT>, 128, 128, 256); break;
     case kF6Tile64: go(gemm_f6_sm<128, 64, OT>, 128, 64, 256); break;
   }
@@ -706,5 +728,9 @@ template void f6_gemm_launch<OutF16>(const int32_t*, int64_t, const int32_t*, in
 template void f6_gemm_launch<OutBF16>(const int32_t*, int64_t, const int32_t*, int64_t, int64_t, const void*, int,
                                       const void*, int, __bf16*, int64_t, const __bf16*, int64_t, int64_t, int64_t,
                                       void*, hipStream_t);
+
+template void f6_gemm_launch<OutF32>(const int32_t*, int64_t, const int32_t*, int64_t, int64_t, const void*, int,
+                                     const void*, int, float*, int64_t, const float*, int64_t, int64_t, int64_t,
+                                     void*, hipStream_t);
 
 }  // namespace qo
