@@ -365,6 +365,14 @@ int qo_pack_int4_to_int32(const int8_t* codes, int64_t codes_ld, int64_t rows, i
                           int32_t* out, int64_t out_ld, void* stream);
 
 /*
+ * qo_pack_int4_to_int32 of the codes clamped to [-8, 7], in one pass: the
+ * weight packing of pack_int4_to_int32_manual (w4a4_flatquant_dynamic.py:43-67)
+ * with its clamp. Arguments and errors as qo_pack_int4_to_int32.
+ */
+int qo_pack_int4_clamped(const int8_t* codes, int64_t codes_ld, int64_t rows, int64_t features,
+                         int32_t* out, int64_t out_ld, void* stream);
+
+/*
  * Unpack int32 words into int8 codes: out[8p + i] = ((word_p >> 4i) & 0xF) - 8.
  *
  * Replaces unpack_int32_to_int4 (int4_matmul/ops.py:48-66).

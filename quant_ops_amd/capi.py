@@ -23,7 +23,7 @@ EXPORTED = ("qo_status_string", "qo_version", "qo_last_error", "qo_set_kernel_ro
             "qo_int4_gemm", "qo_int4_gemm_bias", "qo_int4_gemm_ws", "qo_int4_gemm_workspace_size", "qo_int4_gemm_f6_workspace_bytes",
             "qo_int4_gemm_f6_prepare", "qo_int4_gemm_f6_run", "qo_int4_gemm_f6_operand_bytes",
             "qo_int4_gemm_f6_convert", "qo_int4_gemm_f6_run2", "qo_w4a4_linear_f6w", "qo_w4a4_linear", "qo_w4a4_linear_ws", "qo_w4a4_linear_noalloc", "qo_dequantize_int4",
-            "qo_pack_int4_to_int32", "qo_unpack_int32_to_int4", "qo_transpose_int32")
+            "qo_pack_int4_to_int32", "qo_pack_int4_clamped", "qo_unpack_int32_to_int4", "qo_transpose_int32")
 
 # QO_ROUTE_* bits of qo_set_kernel_routing (include/quant_ops_hip.h)
 ROUTE = {"FQ_GENERIC": 1 << 0, "FQ_NO_WAVE": 1 << 1, "FQ_NO_DUO": 1 << 2, "FQ_NO_FEW": 1 << 3,
@@ -101,7 +101,7 @@ def lib():
                                          c_i64, c_vp, c_int, c_vp, c_vp, c_i64, c_vp]
     L.qo_dequantize_int4.restype = c_int
     L.qo_dequantize_int4.argtypes = [c_vp, c_int, c_vp, c_int, c_i64, c_i64, c_vp, c_vp]
-    for name in ("qo_pack_int4_to_int32", "qo_unpack_int32_to_int4", "qo_transpose_int32"):
+    for name in ("qo_pack_int4_to_int32", "qo_pack_int4_clamped", "qo_unpack_int32_to_int4", "qo_transpose_int32"):
         fn = getattr(L, name)
         fn.restype = c_int
         fn.argtypes = [c_vp, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp]
@@ -396,14 +396,16 @@ def _ld(t):
     return t.stride(0) if t.dim() == 2 and t.shape[0] > 1 else t.shape[-1]
 
 
-def pack_int4_to_int32(codes, out=None, stream=None):
-    """Call ``qo_pack_int4_to_int32``: int8 [rows, F] -> int32 [rows, F/8] (rows may be strided)."""
+def pack_int4_to_int32(codes, out=None, stream=None, clamp=False):
+    """Call ``qo_pack_int4_to_int32`` (``qo_pack_int4_clamped`` with ``clamp``):
+    int8 [rows, F] -> int32 [rows, F/8] (rows may be strided)."""
     assert codes.dtype == torch.int8 and codes.dim() == 2 and codes.stride(1) == 1
     rows, feats = codes.shape
     if out is None:
         out = torch.empty((rows, feats // 8), dtype=torch.int32, device=codes.device)
-    _check(lib().qo_pack_int4_to_int32(ctypes.c_void_p(codes.data_ptr()), _ld(codes), rows, feats,
-                                       ctypes.c_void_p(out.data_ptr()), _ld(out), _stream(stream)))
+    pack = lib().qo_pack_int4_clamped if clamp else lib().qo_pack_int4_to_int32
+    _check(pack(ctypes.c_void_p(codes.data_ptr()), _ld(codes), rows, feats, ctypes.c_void_p(out.data_ptr()), _ld(out),
+                _stream(stream)))
     return out
 
 

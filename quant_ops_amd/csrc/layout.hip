@@ -9,7 +9,10 @@
 //           word p = sum_i ((q[8p + i] + 8) mod 256) << 4i (mod 2^32)
 //           (pack_int4_to_int32, int4_matmul/ops.py:23-45: the int8 add, the
 //           uint8 cast and the int32 shifted sum wrap exactly like this, so
-//           out-of-range codes pack the same way too).
+//           out-of-range codes pack the same way too), or of the codes clamped
+//           to [-8, 7] in the same pass (the linear layer's weights: a clamp of
+//           its own reads and writes every byte once more, 21 us of 37 for
+//           14336 x 4096).
 // * unpack: int32 words [rows, W] -> int8 codes [rows, 8W],
 //           q[8p + i] = ((w >> 4i) & 0xF) - 8 (unpack_int32_to_int4, :48-66).
 // * transpose of 32-bit words [R, C] -> [C, R]: a packed weight stored
@@ -34,7 +37,28 @@ __device__ inline uint32_t pack_word(uint32_t c0, uint32_t c1) {
   return w;
 }
 
+// The same word of the codes clamped to [-8, 7]: bytes as 16-bit halves,
+// q ^ 0x80 = q + 128 unsigned, clamped to 120 .. 135, less 120 = the nibble.
+__device__ inline uint32_t pack_word_clamped(uint32_t c0, uint32_t c1) {
+  typedef unsigned short v2u16 __attribute__((ext_vector_type(2)));
+  const v2u16 lo = {120, 120}, hi = {135, 135};
+  auto two = [&](uint32_t v) -> uint32_t {   // two bytes in 16-bit halves -> their nibble values
+    const v2u16 h = __builtin_bit_cast(v2u16, (v & 0x00FF00FFu) ^ 0x00800080u);
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_elementwise_max(h, lo), hi) - lo);
+  };
+  auto four = [&](uint32_t c) -> uint32_t {   // codes 0 .. 3 -> bits 0 .. 15
+    const uint32_t t = two(c) | (two(c >> 8) << 4);
+    return (t & 0xFFu) | ((t >> 8) & 0xFF00u);
+  };
+  return four(c0) | (four(c1) << 16);
+}
+template <bool CLAMP>
+__device__ inline uint32_t pack_codes(uint32_t c0, uint32_t c1) {
+  return CLAMP ? pack_word_clamped(c0, c1) : pack_word(c0, c1);
+}
+
 // 16 codes (two words) per thread; rows of `words_per_row` words.
+template <bool CLAMP>
 __global__ void __launch_bounds__(256)
 pack_kernel_v16(const int8_t* __restrict__ codes, int64_t codes_ld, int64_t rows, int64_t pairs_per_row,
                 int32_t* __restrict__ out, int64_t out_ld) {
@@ -42,12 +66,14 @@ pack_kernel_v16(const int8_t* __restrict__ codes, int64_t codes_ld, int64_t rows
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
     const int64_t r = i / pairs_per_row, p = i - r * pairs_per_row;
     const v4i c = *reinterpret_cast<const v4i*>(codes + r * codes_ld + 16 * p);
-    const v2i w = {(int)pack_word((uint32_t)c[0], (uint32_t)c[1]), (int)pack_word((uint32_t)c[2], (uint32_t)c[3])};
+    const v2i w = {(int)pack_codes<CLAMP>((uint32_t)c[0], (uint32_t)c[1]),
+                   (int)pack_codes<CLAMP>((uint32_t)c[2], (uint32_t)c[3])};
     __builtin_nontemporal_store(w, reinterpret_cast<v2i*>(out + r * out_ld + 2 * p));
   }
 }
 
 // One word per thread, byte loads (any alignment).
+template <bool CLAMP>
 __global__ void __launch_bounds__(256)
 pack_kernel_any(const int8_t* __restrict__ codes, int64_t codes_ld, int64_t rows, int64_t words_per_row,
                 int32_t* __restrict__ out, int64_t out_ld) {
@@ -61,7 +87,7 @@ pack_kernel_any(const int8_t* __restrict__ codes, int64_t codes_ld, int64_t rows
       c0 |= (uint32_t)src[j] << (8 * j);
       c1 |= (uint32_t)src[4 + j] << (8 * j);
     }
-    out[r * out_ld + p] = (int)pack_word(c0, c1);
+    out[r * out_ld + p] = (int)pack_codes<CLAMP>(c0, c1);
   }
 }
 
@@ -161,21 +187,18 @@ static unsigned grid_for(int64_t items) {
   return (unsigned)(blocks < 1 ? 1 : blocks);
 }
 
-
-}  // namespace qo
-
-extern "C" int qo_pack_int4_to_int32(const int8_t* codes, int64_t codes_ld, int64_t rows, int64_t features,
-                                     int32_t* out, int64_t out_ld, void* stream) {
-  using namespace qo;
+template <bool CLAMP>
+static int pack_codes_entry(const char* who, const int8_t* codes, int64_t codes_ld, int64_t rows, int64_t features,
+                            int32_t* out, int64_t out_ld, void* stream) {
   if (rows < 0 || features < 0 || features % 8 != 0 || (rows > 1 && (codes_ld < features || out_ld < features / 8))) {
-    qo_set_error("qo_pack_int4_to_int32: invalid sizes rows=%lld features=%lld (features must be a multiple of 8) "
-                 "codes_ld=%lld out_ld=%lld", (long long)rows, (long long)features, (long long)codes_ld,
+    qo_set_error("%s: invalid sizes rows=%lld features=%lld (features must be a multiple of 8) "
+                 "codes_ld=%lld out_ld=%lld", who, (long long)rows, (long long)features, (long long)codes_ld,
                  (long long)out_ld);
     return QO_ERR_SHAPE;
   }
   if (rows == 0 || features == 0) return QO_OK;
   if (!codes || !out) {
-    qo_set_error("qo_pack_int4_to_int32: NULL pointer argument");
+    qo_set_error("%s: NULL pointer argument", who);
     return QO_ERR_NULL_POINTER;
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -184,14 +207,26 @@ extern "C" int qo_pack_int4_to_int32(const int8_t* codes, int64_t codes_ld, int6
                    (rows == 1 || (codes_ld % 16 == 0 && out_ld % 2 == 0));
   if (vec) {
     const int64_t pairs = features / 16;
-    launch(pack_kernel_v16, dim3(grid_for(rows * pairs)), dim3(256), 0, s, codes, codes_ld, rows, pairs,
+    launch(pack_kernel_v16<CLAMP>, dim3(grid_for(rows * pairs)), dim3(256), 0, s, codes, codes_ld, rows, pairs,
                        out, out_ld);
   } else {
     const int64_t wpr = features / 8;
-    launch(pack_kernel_any, dim3(grid_for(rows * wpr)), dim3(256), 0, s, codes, codes_ld, rows, wpr, out,
+    launch(pack_kernel_any<CLAMP>, dim3(grid_for(rows * wpr)), dim3(256), 0, s, codes, codes_ld, rows, wpr, out,
                        out_ld);
   }
-  return launch_result("qo_pack_int4_to_int32");
+  return launch_result(who);
+}
+
+}  // namespace qo
+
+extern "C" int qo_pack_int4_to_int32(const int8_t* codes, int64_t codes_ld, int64_t rows, int64_t features,
+                                     int32_t* out, int64_t out_ld, void* stream) {
+  return qo::pack_codes_entry<false>("qo_pack_int4_to_int32", codes, codes_ld, rows, features, out, out_ld, stream);
+}
+
+extern "C" int qo_pack_int4_clamped(const int8_t* codes, int64_t codes_ld, int64_t rows, int64_t features,
+                                    int32_t* out, int64_t out_ld, void* stream) {
+  return qo::pack_codes_entry<true>("qo_pack_int4_clamped", codes, codes_ld, rows, features, out, out_ld, stream);
 }
 
 extern "C" int qo_unpack_int32_to_int4(const int32_t* words, int64_t words_ld, int64_t rows, int64_t nwords,

@@ -43,6 +43,11 @@ def _scale_dtype(s: torch.Tensor) -> torch.Tensor:
 def prepare_w4a4_weight(weight_codes: torch.Tensor) -> torch.Tensor:
     """int4 weight codes stored as integers [out, in] -> packed int32 [out, in/8]."""
     assert weight_codes.dim() == 2 and weight_codes.shape[1] % 8 == 0, "[out, in] with in % 8 == 0"
+    if weight_codes.is_cuda and weight_codes.dtype == torch.int8:
+        _loader.require_kernels("prepare_w4a4_weight")
+        from . import capi
+        return capi.pack_int4_to_int32(weight_codes if weight_codes.stride(1) == 1 else weight_codes.contiguous(),
+                                       clamp=True)
     return pack_int4_to_int32(weight_codes.clamp(-8, 7).to(torch.int8))
 
 

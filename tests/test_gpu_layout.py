@@ -140,3 +140,16 @@ def test_w4a4_linear_gpu(gpu, tokens):
     assert int(d.max()) <= 1 and float((d != 0).float().mean()) <= 1e-3
     ref = oi4.int4_matmul_pytorch(q.cpu(), wp.cpu().t(), s.cpu(), sw, out_dtype=torch.bfloat16) + bias
     assert torch.equal(y.cpu(), ref)
+
+
+@pytest.mark.parametrize("rows,feats,stride", [(1, 8, 8), (3, 24, 24), (5, 64, 64), (7, 48, 61), (130, 4096, 4096)])
+def test_pack_clamped_every_int8(gpu, rows, feats, stride):
+    """prepare_w4a4_weight of int8 codes (clamp and pack in one kernel, whole
+    16-byte and byte-wise forms) against the clamp and the oracle's packing, for
+    every int8 value."""
+    g = torch.Generator().manual_seed(rows + feats)
+    wide = torch.randint(-128, 128, (rows, stride), generator=g, dtype=torch.int8)
+    wide.view(-1)[:256] = torch.arange(-128, 128).to(torch.int8)[: wide.numel()]
+    codes = wide[:, :feats]
+    got = qo.prepare_w4a4_weight(wide.to(gpu)[:, :feats]).cpu()
+    assert torch.equal(got, qo.pack_int4_to_int32(codes.clamp(-8, 7)))
