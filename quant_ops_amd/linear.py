@@ -46,8 +46,8 @@ def prepare_w4a4_weight(weight_codes: torch.Tensor) -> torch.Tensor:
     if weight_codes.is_cuda and weight_codes.dtype == torch.int8:
         _loader.require_kernels("prepare_w4a4_weight")
         from . import capi
-        return capi.pack_int4_to_int32(weight_codes if weight_codes.stride(1) == 1 else weight_codes.contiguous(),
-                                       clamp=True)
+        rows_apart = weight_codes.stride(1) == 1 and weight_codes.stride(0) >= weight_codes.shape[1]   # not an expanded row
+        return capi.pack_int4_to_int32(weight_codes if rows_apart else weight_codes.contiguous(), clamp=True)
     return pack_int4_to_int32(weight_codes.clamp(-8, 7).to(torch.int8))
 
 

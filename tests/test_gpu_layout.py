@@ -153,3 +153,17 @@ def test_pack_clamped_every_int8(gpu, rows, feats, stride):
     codes = wide[:, :feats]
     got = qo.prepare_w4a4_weight(wide.to(gpu)[:, :feats]).cpu()
     assert torch.equal(got, qo.pack_int4_to_int32(codes.clamp(-8, 7)))
+
+
+@pytest.mark.parametrize("rows,feats,form", [(5, 64, "expanded"), (5, 24, "expanded"), (6, 64, "overlapping"),
+                                             (16, 40, "columns")])
+def test_prepare_weight_strides(gpu, rows, feats, form):
+    """Codes whose rows share memory (one row expanded, overlapping windows) or
+    run down the columns pack as their contiguous copy does."""
+    g = torch.Generator().manual_seed(rows * feats)
+    base = torch.randint(-128, 128, (rows * feats,), generator=g, dtype=torch.int8)
+    view = {"expanded": lambda t: t[:feats].expand(rows, feats),
+            "overlapping": lambda t: t.as_strided((rows, feats), (8, 1)),
+            "columns": lambda t: t.view(feats, rows).t()}[form]
+    got = qo.prepare_w4a4_weight(view(base.to(gpu))).cpu()
+    assert torch.equal(got, qo.pack_int4_to_int32(view(base).contiguous().clamp(-8, 7)))
