@@ -414,14 +414,20 @@ gemm_f6_pp2(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int 
 // multiplies stage t, so a stage costs one barrier: it says that stage t + 1
 // has landed and that every wave holds stage t in registers, which frees its
 // slot for the copies of stage t + 3.
+//
+// SPLIT: eight waves, waves 4 .. 7 the odd k-blocks of the same tile on a ring
+// of their own, where a CU has one tile only: one wave per SIMD leaves its LDS
+// reads, MFMAs and barriers in a row (345 ns per 128 x 64 stage), two groups
+// overlap theirs (about 255 ns a stage). The odd blocks' sums go to the first group through LDS; both
+// are integers below 2^23, so their float32 sum is exact.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, class OT>
-__global__ void __launch_bounds__(256, 2)
+template <int BM, int BN, class OT, bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? 512 : 256, 2)
 gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int pr_a, int pr_b, int nk,
            const void* __restrict__ sa, int sad, const void* __restrict__ sb, int sbd,
            typename OT::T* __restrict__ out, int64_t ldc, const typename OT::T* __restrict__ bias, int M, int N,
            int tiles_m) {
-  constexpr int W = 4, STAGES = 3;
+  constexpr int W = 4, STAGES = 3, GROUPS = SPLIT ? 2 : 1;
   using S = F6Stage<BM, BN>;
   using T = typename OT::T;
   constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16, QA = FM / 2, QB = FN / 2;
@@ -429,14 +435,17 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
   constexpr bool kF32 = sizeof(T) == 4;   // float32 outputs are stored from registers, 16-bit ones through LDS
   static_assert(S::A_DMA % W == 0 && FM % 2 == 0 && FN % 2 == 0 && BM <= 128 && BN <= 128, "tile");
   constexpr int C_PITCH = BN * 2 + 16;
-  __shared__ __align__(16) unsigned char ring[STAGES * S::BYTES];
+  constexpr int RING = STAGES * S::BYTES;   // a group's
+  __shared__ __align__(16) unsigned char ring[GROUPS * RING];
   static_assert(PER * (STAGES - 1) < 64, "vmcnt range");
-  static_assert(BM * C_PITCH <= STAGES * S::BYTES, "staged output");
+  static_assert(BM * C_PITCH <= RING && (!SPLIT || BM * BN * 4 <= RING), "staged output and partial sums");
   __shared__ __align__(16) float s_sa[BM];
   __shared__ __align__(16) float s_sb[BN];
   __shared__ __align__(16) float s_bias[BN];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
+  const int grp = SPLIT ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+  const int ns = SPLIT ? (nk - grp + 1) >> 1 : nk;   // this group's stages: stage t is k-block GROUPS t + grp
   const int wm = wave >> 1, wn = wave & 1;
   const int li = lane & 15, lg = lane >> 4;
 
@@ -472,8 +481,10 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
     }
     dst[t] = __builtin_amdgcn_readfirstlane((uint32_t)(1024 * i));
   }
-  const uint32_t ring0 = lds_addr(ring);
-  auto issue = [&](int ks, int slot) __attribute__((always_inline)) {
+  unsigned char* const my_ring = ring + grp * RING;
+  const uint32_t ring0 = lds_addr(my_ring);
+  auto issue = [&](int t0, int slot) __attribute__((always_inline)) {
+    const int ks = GROUPS * t0 + grp;
     const uint32_t base = ring0 + slot * S::BYTES;
     const uint8_t* ab = a_base + (int64_t)ks * kF6Pair;
     const uint8_t* bb = b_base + (int64_t)ks * kF6Pair;
@@ -489,7 +500,7 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
   };
   auto load_regs = [&](auto setc, int slot) __attribute__((always_inline)) {
     constexpr int H = decltype(setc)::value;
-    const unsigned char* base = ring + slot * S::BYTES + 16 * lane;
+    const unsigned char* base = my_ring + slot * S::BYTES + 16 * lane;
 #pragma unroll
     for (int q = 0; q < QA; ++q) ap[H][q] = pair_at(base + (wm * QA + q) * kF6Pair);
 #pragma unroll
@@ -522,8 +533,8 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
 
 #pragma unroll
   for (int t = 0; t < STAGES; ++t)
-    if (t < nk) issue(t, t);
-  gemm_wait_groups<PER, STAGES - 1>(nk - 1);
+    if (t < ns) issue(t, t);
+  gemm_wait_groups<PER, STAGES - 1>(ns - 1);
   raw_barrier();
   load_regs(std::integral_constant<int, 0>{}, 0);
 
@@ -531,24 +542,27 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
   auto stage = [&](int t, auto setc) __attribute__((always_inline)) {
     constexpr int H = decltype(setc)::value;
     __builtin_amdgcn_sched_barrier(0);
-    gemm_wait_groups<PER, STAGES - 2>(nk - 2 - t);   // stage t + 1 has landed (the later ones may be in flight)
+    gemm_wait_groups<PER, STAGES - 2>(ns - 2 - t);   // stage t + 1 has landed (the later ones may be in flight)
     __builtin_amdgcn_s_waitcnt(0xC07F);     // lgkmcnt(0): stage t is in this wave's registers
     raw_barrier();
     __builtin_amdgcn_sched_barrier(0);
     const int next = slot == STAGES - 1 ? 0 : slot + 1;
-    if (t + STAGES < nk) issue(t + STAGES, slot);
-    if (t + 1 < nk) load_regs(std::integral_constant<int, 1 - H>{}, next);
+    if (t + STAGES < ns) issue(t + STAGES, slot);
+    if (t + 1 < ns) load_regs(std::integral_constant<int, 1 - H>{}, next);
+    if (!SPLIT || t < ns) {   // the second group may have one stage less
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-            half(bp[H][j >> 1], j & 1), half(ap[H][i >> 1], i & 1), acc[i][j], 2, 2, 0, 130, 0, 130);
+        for (int i = 0; i < FM; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+              half(bp[H][j >> 1], j & 1), half(ap[H][i >> 1], i & 1), acc[i][j], 2, 2, 0, 130, 0, 130);
+    }
     slot = next;
   };
-  for (int t = 0; t < nk; t += 2) {
+  const int stages = SPLIT ? (nk + 1) >> 1 : nk;   // of the first group: every wave meets every barrier
+  for (int t = 0; t < stages; t += 2) {
     stage(t, std::integral_constant<int, 0>{});
-    if (t + 1 < nk) stage(t + 1, std::integral_constant<int, 1>{});
+    if (t + 1 < stages) stage(t + 1, std::integral_constant<int, 1>{});
   }
 
   // acc[i][j][r] is row wm * WM + 16 i + li, column wn * WN + 16 j + 4 lg + r;
@@ -562,43 +576,62 @@ gemm_f6_sm(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ b6, int p
     else s_bias[tid - 128] = (float)__builtin_bit_cast(T, (uint16_t)rbias);
   }
   __syncthreads();   // also: no wave reads the ring any more
+  unsigned char* const c_tile = ring + (GROUPS - 1) * RING;   // apart from the partial sums
+  if constexpr (SPLIT) {
+    v4f* const part = reinterpret_cast<v4f*>(ring) + (tid & 255);
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) part[256 * (i * FN + j)] = acc[i][j];
+    }
+    lds_barrier();
+    if (grp == 0) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] += part[256 * (i * FN + j)];
+    }
+  }
   const bool vec = kF32 && (uintptr_t)out % 16 == 0 && ldc % 4 == 0;
+  if (grp == 0) {
 #pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int row = wm * WM + 16 * i + li;
-    const float sav = s_sa[row];
+    for (int i = 0; i < FM; ++i) {
+      const int row = wm * WM + 16 * i + li;
+      const float sav = s_sa[row];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int c = wn * WN + 16 * j + 4 * lg;
-      const v4f sbv = *reinterpret_cast<const v4f*>(s_sb + c);
-      T v[4];
+      for (int j = 0; j < FN; ++j) {
+        const int c = wn * WN + 16 * j + 4 * lg;
+        const v4f sbv = *reinterpret_cast<const v4f*>(s_sb + c);
+        T v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = OT::cvt((acc[i][j][r] * sav) * sbv[r]);
-      if (bias) {
-        const v4f bb = *reinterpret_cast<const v4f*>(s_bias + c);
+        for (int r = 0; r < 4; ++r) v[r] = OT::cvt((acc[i][j][r] * sav) * sbv[r]);
+        if (bias) {
+          const v4f bb = *reinterpret_cast<const v4f*>(s_bias + c);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = OT::cvt((float)v[r] + bb[r]);
-      }
-      if constexpr (kF32) {
-        const int m = m0 + row, n = n0 + c;
-        if (m >= M) continue;
-        T* const o = out + (int64_t)m * ldc + n;
-        if (vec && n + 3 < N) {
-          *reinterpret_cast<v4f*>(o) = v4f{v[0], v[1], v[2], v[3]};
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < N) o[r] = v[r];
+          for (int r = 0; r < 4; ++r) v[r] = OT::cvt((float)v[r] + bb[r]);
         }
-      } else {
-        *reinterpret_cast<v2i*>(ring + row * C_PITCH + 2 * c) =
-            v2i{(int)(out_bits<OT>(v[0]) | out_bits<OT>(v[1]) << 16), (int)(out_bits<OT>(v[2]) | out_bits<OT>(v[3]) << 16)};
+        if constexpr (kF32) {
+          const int m = m0 + row, n = n0 + c;
+          if (m >= M) continue;
+          T* const o = out + (int64_t)m * ldc + n;
+          if (vec && n + 3 < N) {
+            *reinterpret_cast<v4f*>(o) = v4f{v[0], v[1], v[2], v[3]};
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n + r < N) o[r] = v[r];
+          }
+        } else {
+          *reinterpret_cast<v2i*>(c_tile + row * C_PITCH + 2 * c) =
+              v2i{(int)(out_bits<OT>(v[0]) | out_bits<OT>(v[1]) << 16), (int)(out_bits<OT>(v[2]) | out_bits<OT>(v[3]) << 16)};
+        }
       }
     }
   }
   if constexpr (!kF32) {
     lds_barrier();
-    copy_out_c<BM, BN, 256, OT, true>(ring, C_PITCH, out, ldc, M, N, m0, n0, tid);
+    copy_out_c<BM, BN, 256 * GROUPS, OT, true>(c_tile, C_PITCH, out, ldc, M, N, m0, n0, tid);
   }
 }
 
@@ -638,10 +671,16 @@ namespace {
 // but leaves more CUs idle. Per stage, measured at 4096 columns x 14336: 256-row
 // tiles 740 (850 with every CU busy, 256 columns wide), 128 x 128 430 for one
 // workgroup on a CU and 700 for two, 128 x 64 345 and 480; per round 8 us and 4 us.
+// Split tiles (one per CU, two groups of waves) take 670 and 510 for a pair of
+// stages, and 1 us more a round for the sums' exchange: they win where a round
+// leaves CUs with one tile and K is 1536 or more. Kernel alone, unsplit -> split:
+// 512 x 4096 x 14336 38.6 -> 33.8 us, 640 x 3584 x 18944 61.1 -> 49.2 us,
+// 400 x 8192 x 28672 94.6 -> 80.2 us, 1024 x 4096 x 14336 49.7 -> 42.1 us,
+// 300 x 2048 x 2048 7.7 -> 7.4 us.
 // With 256-row tiles alone M = 512 took 83.7 us there (38 tiles on 256 CUs), on
 // 128 x 64 it takes 40 us; 512 x 14336 x 4096 33 -> 25 us on 128 x 128; 2048 x
 // 4096 x 4096 34 -> 25 us; 2048 x 14336 x 4096 keeps 256 x 224 (87 us against 94).
-enum F6Tile { kF6Tile224, kF6Tile256, kF6Tile128, kF6Tile64 };
+enum F6Tile { kF6Tile224, kF6Tile256, kF6Tile128, kF6Tile64, kF6Split128, kF6Split64 };
 F6Tile f6_tile(int64_t M, int64_t N, int64_t K, bool f32) {
   const int64_t cus = device_cu_count(), nk = (K + 127) / 128;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -650,10 +689,11 @@ F6Tile f6_tile(int64_t M, int64_t N, int64_t K, bool f32) {
     const int64_t full = t / (2 * cus), rest = t % (2 * cus);
     return full * (nk * two + 4000) + (rest == 0 ? 0 : nk * (rest <= cus ? one : two) + 4000);
   };
-  const int64_t est[4] = {wide(tiles(256, 224), 745), wide(tiles(256, 256), 850), pair(tiles(128, 128), 430, 700),
-                          pair(tiles(128, 64), 345, 480)};
+  auto split = [&](int64_t t, int64_t stage) { return (t + cus - 1) / cus * ((nk + 1) / 2 * stage + 5000); };
+  const int64_t est[6] = {wide(tiles(256, 224), 745), wide(tiles(256, 256), 850), pair(tiles(128, 128), 430, 700),
+                          pair(tiles(128, 64), 345, 480), split(tiles(128, 128), 670), split(tiles(128, 64), 510)};
   int best = f32 ? 2 : 0;   // the 256-row kernel stages 16-bit values
-  for (int i = best + 1; i < 4; ++i)
+  for (int i = best + 1; i < 6; ++i)
     if (est[i] < est[best]) best = i;
   return (F6Tile)best;
 }
@@ -701,8 +741,10 @@ void f6_run2(const void* a6v, const void* b6v, const void* sa, int sad, const vo
     case kF6Tile256:
       if constexpr (!kF32) go(gemm_f6_pp2<256, 256, OT>, 256, 256, 512);
       break;
-    case kF6Tile128: go(gemm_f6_sm<128, 128, OT>, 128, 128, 256); break;
-    case kF6Tile64: go(gemm_f6_sm<128, 64, OT>, 128, 64, 256); break;
+    case kF6Tile128: go(gemm_f6_sm<128, 128, OT, false>, 128, 128, 256); break;
+    case kF6Tile64: go(gemm_f6_sm<128, 64, OT, false>, 128, 64, 256); break;
+    case kF6Split128: go(gemm_f6_sm<128, 128, OT, true>, 128, 128, 512); break;
+    case kF6Split64: go(gemm_f6_sm<128, 64, OT, true>, 128, 64, 512); break;
   }
 }
 

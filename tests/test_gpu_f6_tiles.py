@@ -40,3 +40,31 @@ def test_f6_tile_equals_integer_route(gpu, m, n, k, out_dtype, bias):
         ref = capi.int4_gemm(a, b, sa, sb, out_dtype=out_dtype, bias=bv)
     torch.cuda.synchronize()
     assert torch.equal(out, ref) and bool((wide[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("out_dtype,bias", [(torch.float16, False), (torch.bfloat16, True), (torch.float32, True)])
+@pytest.mark.parametrize("m,n,k", [
+    (300, 333, 2048),       # 128 x 64 by two groups of waves, 16 k-blocks: eight for each
+    (300, 333, 2056),       # 17: the second group has one less
+    (257, 4097, 2312),      # 128 x 64, odd N, 19 k-blocks
+    (300, 11001, 3080),     # 128 x 128 by two groups, 25 k-blocks
+    (511, 4100, 65536),     # the largest sums
+])
+def test_f6_split_tile_equals_integer_route(gpu, m, n, k, out_dtype, bias):
+    """Tiles whose k-blocks two groups of waves share, against the integer route bit for bit."""
+    print(f"[gpu-f6-split] {m}x{n}x{k} {out_dtype} bias={bias}", flush=True)
+    g = torch.Generator().manual_seed(m + k)
+    a = torch.randint(-2 ** 31, 2 ** 31, (m, k // 8), generator=g, dtype=torch.int32).to(gpu)
+    b = torch.randint(-2 ** 31, 2 ** 31, (n, k // 8), generator=g, dtype=torch.int32).to(gpu).t()
+    if k == 65536:
+        a[0], b[:, 0] = 0, 0   # every product 64: the sum 2^22
+    sa = (0.01 + torch.rand(m, generator=g)).to(gpu)
+    sb = (0.001 * torch.rand(n, generator=g)).to(gpu).half()
+    bv = wl.uniform(n, -1.0, 1.0, 7, out_dtype).to(gpu) if bias else None
+    if out_dtype == torch.float32 and n % 4 == 0 and k % 128 == 0:
+        pytest.skip("float32 outputs of whole rows and stages stay on the integer route")
+    out = capi.int4_gemm(a, b, sa, sb, out_dtype=out_dtype, bias=bv, workspace=True)
+    with capi.kernel_routing("GEMM_NO_F6"):
+        ref = capi.int4_gemm(a, b, sa, sb, out_dtype=out_dtype, bias=bv)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
