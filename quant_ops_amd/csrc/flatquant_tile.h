@@ -78,10 +78,12 @@ template <class T, int CH>
 struct FqTileRows {
   v4i v[CH];
   T tail;
-  __device__ void load(const T* __restrict__ src, int elems, int tid, int nt) {
+  __host__ __device__ void load(const T* __restrict__ src, int elems, int tid, int nt) {
     const int chunks = elems >> 3;
+    if (chunks > 0) {   // a 2 x 2 matrix is all tail
 #pragma unroll
-    for (int i = 0; i < CH; ++i) v[i] = reinterpret_cast<const v4i*>(src)[max(min(tid + i * nt, chunks - 1), 0)];
+      for (int i = 0; i < CH; ++i) v[i] = reinterpret_cast<const v4i*>(src)[min(tid + i * nt, chunks - 1)];
+    }
     tail = src[min(8 * chunks + tid, elems - 1)];
   }
   template <bool EVEN>
