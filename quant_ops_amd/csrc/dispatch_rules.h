@@ -1,0 +1,28 @@
+// Rules that choose a kernel from sizes and types. Plain functions of their
+// arguments (the number of CUs among them), so that the CPU tests can run them.
+#pragma once
+
+#include <stdint.h>
+
+namespace qo {
+
+// fp16 / bf16 shapes and token counts at which fq_mfma_kernel's zero-padded
+// fragments are faster than fq_tile_kernel: where one round of tile workgroups
+// fills every CU (four of 56 x 64, two of the others), their set-ups share the
+// CU's LDS and the LDS-DMA copies of fq_mfma_kernel do not; and 64 x 80 fp16
+// beyond two tokens per CU, whose 99 registers let two workgroups of five waves
+// share a CU and not three (bf16: 93, three). Measured on 256 CUs, kernel alone,
+// packed codes, fp16, tile -> mfma: 80 x 112, 300 tokens 10.6 -> 9.4 us, 512
+// tokens 11.1 -> 9.9 us (256 tokens 8.0 against 8.3, 600 tokens 16.3 against
+// 21.1); 72 x 96, 512 tokens 10.1 -> 9.8 us; 64 x 112, 512 tokens 9.1 -> 8.7 us
+// (bf16 the same on both); 56 x 64, 1021 tokens 8.5 -> 8.1 us; 64 x 80, 1024
+// tokens 13.6 -> 9.8 us, 4096 tokens 27.7 -> 21.3 us (bf16 21.2 against 24.4).
+inline bool fq_padded_mfma(int M, int N, int64_t tokens, bool f16, int64_t cus) {
+  const int64_t per_cu = (tokens + cus - 1) / cus;
+  if (M == 56 && N == 64) return per_cu == 4;
+  if (M == 64 && N == 80) return f16 && per_cu > 2;
+  if ((M == 64 && N == 112) || (M == 72 && N == 96) || (M == 80 && N == 112)) return per_cu == 2;
+  return false;
+}
+
+}  // namespace qo

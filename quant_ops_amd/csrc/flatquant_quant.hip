@@ -38,6 +38,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "dispatch_rules.h"
 #include "flatquant_common.h"
 
 namespace qo {
@@ -2278,6 +2279,13 @@ static int dispatch_mfma(int M, int N, const void* x, int64_t tokens, int64_t x_
                                                 stream);
   QO_FQ_CASE_NV(2, 2, 48)    // 32 x 48   (hidden 1536)
   QO_FQ_CASE_NV(4, 3, 88)    // 64 x 88   (hidden 5632)
+  const bool clip_pos = clip > 0.f && clip <= 3.4e38f;   // fq_tile_kernel takes the scale from max |Y|
+  const bool padded = !clip_pos || fq_padded_mfma(M, N, tokens, std::is_same<DT, F16T>::value, device_cu_count());
+  if (padded) {
+    QO_FQ_CASE_NV(4, 3, 80)    // 64 x 80   (hidden 5120)
+    QO_FQ_CASE_NV(4, 4, 112)   // 64 x 112  (hidden 7168)
+    QO_FQ_CASE_NV(5, 4, 112)   // 80 x 112  (hidden 8960)
+  }
 #undef QO_FQ_CASE_NV
   // heights that are not a multiple of 16: computed zero-padded to 16 MB
 #define QO_FQ_CASE_MV(MB_, NP_, MV_)                                                                          \
@@ -2285,6 +2293,10 @@ static int dispatch_mfma(int M, int N, const void* x, int64_t tokens, int64_t x_
     return launch_mfma<DT, MB_, NP_, PACK, 32 * (NP_), MV_>(x, tokens, x_ld, left, right, clip, out_codes,    \
                                                             out_scales, stream);
   QO_FQ_CASE_MV(3, 2, 40)    // 40 x 64   (hidden 2560)
+  if (padded) {
+    QO_FQ_CASE_MV(4, 2, 56)    // 56 x 64   (hidden 3584)
+    QO_FQ_CASE_MV(5, 3, 72)    // 72 x 96   (hidden 6912)
+  }
 #undef QO_FQ_CASE_MV
   // Every other shape (scale from max |Y|: clip > 0). The shapes above are those
   // where fq_mfma_kernel was the faster of the two: whole fragments, which X's
@@ -2292,7 +2304,7 @@ static int dispatch_mfma(int M, int N, const void* x, int64_t tokens, int64_t x_
   // 24 us against 27, 128 x 224 140 against 151), and small padded ones (40 x 64
   // 14.2 against 15.5). Padded widths and heights beyond those, and 128 x 160,
   // 128 x 192, 144 x 192 and 160 x 160, run 5 to 60 % faster on fq_tile_kernel.
-  if (clip > 0.f && clip <= 3.4e38f &&
+  if (clip_pos &&
       launch_tile<DT>(x, tokens, x_ld, left, right, M, N, clip, PACK ? 1 : 0, out_codes, out_scales, stream))
     return QO_OK;
   *handled = false;

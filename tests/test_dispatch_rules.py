@@ -1,0 +1,45 @@
+"""CPU check of the rules that choose a kernel (quant_ops_amd/csrc/dispatch_rules.h),
+compiled as they are, at the lines that their measurements drew (256 CUs)."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CUS = 256
+
+SOURCE = r"""
+#include "dispatch_rules.h"
+extern "C" int padded_mfma(int M, int N, int64_t tokens, int f16, int64_t cus) {
+  return qo::fq_padded_mfma(M, N, tokens, f16 != 0, cus);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, lib = d / "rules.cpp", d / "librules.so"
+    src.write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{ROOT}/quant_ops_amd/csrc", str(src), "-o",
+                    str(lib)], check=True)
+    return ctypes.CDLL(str(lib))
+
+
+@pytest.mark.parametrize("m,n,f16,first,last", [
+    (56, 64, True, 769, 1024), (56, 64, False, 769, 1024),
+    (64, 80, True, 513, None), (64, 112, True, 257, 512), (72, 96, False, 257, 512), (80, 112, False, 257, 512),
+])
+def test_padded_shapes_on_the_fragment_kernel(rules, m, n, f16, first, last):
+    def takes(tokens):
+        return bool(rules.padded_mfma(m, n, ctypes.c_int64(tokens), int(f16), ctypes.c_int64(CUS)))
+
+    assert not takes(1) and not takes(first - 1) and takes(first)
+    assert takes(8192) if last is None else takes(last) and not takes(last + 1) and not takes(8192)
+
+
+def test_other_shapes_stay_on_the_tile_kernel(rules):
+    for m, n, f16 in [(64, 80, 0), (128, 144, 1), (86, 128, 1), (108, 128, 0), (76, 128, 1), (96, 96, 1), (112, 64, 1)]:
+        for tokens in (1, 256, 300, 512, 600, 1024, 4096):
+            assert not rules.padded_mfma(m, n, ctypes.c_int64(tokens), f16, ctypes.c_int64(CUS)), (m, n, f16, tokens)
