@@ -25,4 +25,21 @@ inline bool fq_padded_mfma(int M, int N, int64_t tokens, bool f16, int64_t cus) 
   return false;
 }
 
+// Quantize calls of a few features and fewer tokens than CUs that the generic
+// kernel finishes sooner than fq_tile_kernel / fq_f32_kernel, whose set-up
+// (operand fragments of 16 rows and columns) is then most of the time. Its
+// fast form needs M and N to be multiples of 4, and packing costs it an
+// exchange. Measured, 1 token, int8 codes, fragment kernel -> generic: float32
+// 4 x 4 4.7 -> 3.8 us, 8 x 8 4.5 -> 4.0 us, 8 x 12 4.4 -> 4.1 us (12 x 12 4.4
+// against 4.3); 4 x 6 4.8 -> 4.5 us; fp16 4 x 8 4.5 -> 4.2 us, 8 x 8 4.4 -> 4.3
+// us (8 x 12 the same, 5 x 8 4.3 against 6.3); packed float32 4 x 4 4.7 -> 4.3 us
+// (4 x 8 the same). At 256 tokens the fragment kernels win from 24 features.
+inline bool fq_generic_few(int M, int N, int64_t tokens, bool f32, bool pack, int64_t cus) {
+  const int64_t F = (int64_t)M * N;
+  if (tokens >= cus) return false;
+  if (pack) return f32 && F <= 16;
+  if (M % 4 == 0 && N % 4 == 0) return F <= (f32 ? 96 : 64);
+  return f32 && F <= 32;
+}
+
 }  // namespace qo

@@ -20,11 +20,13 @@
 //                       streamed into LDS by LDS-DMA one token group ahead (two
 //                       stages, one where two do not fit); L is resident in VGPRs
 //                       or LDS, R in VGPRs.
-//  * fq_tile_kernel   — (flatquant_tile.h) fp16 / bf16, every other shape with N
-//                       even up to 256 and M up to 176.
+//  * fq_tile_kernel   — (flatquant_tile.h) fp16 / bf16, the other shapes with N
+//                       even up to 256 and M up to 176 that are not much taller
+//                       than wide (its table of instances).
 //  * fq_f32_kernel    — (flatquant_f32.hip) fp32, N up to 256 (even when packing)
 //                       and M up to 128, where X and L fit in LDS: the generic
 //                       kernel's sums, bit for bit, on the float32 matrix cores.
+//  (which of them where: the rules in dispatch_rules.h)
 //  * fq_generic_kernel — any M, N, D in {fp32, fp16, bf16}; VALU fp32 FMA with the
 //                       same rounding points. Used for shapes the MFMA kernels
 //                       do not cover, X and Z in LDS.
@@ -2304,7 +2306,7 @@ static int dispatch_mfma(int M, int N, const void* x, int64_t tokens, int64_t x_
   // 24 us against 27, 128 x 224 140 against 151), and small padded ones (40 x 64
   // 14.2 against 15.5). Padded widths and heights beyond those, and 128 x 160,
   // 128 x 192, 144 x 192 and 160 x 160, run 5 to 60 % faster on fq_tile_kernel.
-  if (clip_pos &&
+  if (clip_pos && !fq_generic_few(M, N, tokens, false, PACK, device_cu_count()) &&
       launch_tile<DT>(x, tokens, x_ld, left, right, M, N, clip, PACK ? 1 : 0, out_codes, out_scales, stream))
     return QO_OK;
   *handled = false;
@@ -2376,6 +2378,7 @@ static int run_quantize(const void* x, int64_t tokens, int64_t x_ld, const void*
     // 16-byte loads of X rows and stores of codes; scale from max |Y| (clip > 0)
     const bool aligned = (uintptr_t)x % 16 == 0 && x_ld % 4 == 0 && (uintptr_t)out_codes % 16 == 0;
     if (allow_mfma && aligned && clip > 0.f && clip <= 3.4e38f &&
+        !fq_generic_few(M, N, tokens, true, PACK, device_cu_count()) &&
         launch_f32(reinterpret_cast<const float*>(x), tokens, x_ld, reinterpret_cast<const float*>(left),
                    reinterpret_cast<const float*>(right), M, N, clip, PACK ? 1 : 0, out_codes, out_scales, stream))
       return QO_OK;

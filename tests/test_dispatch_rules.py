@@ -14,6 +14,9 @@ SOURCE = r"""
 extern "C" int padded_mfma(int M, int N, int64_t tokens, int f16, int64_t cus) {
   return qo::fq_padded_mfma(M, N, tokens, f16 != 0, cus);
 }
+extern "C" int generic_few(int M, int N, int64_t tokens, int f32, int pack, int64_t cus) {
+  return qo::fq_generic_few(M, N, tokens, f32 != 0, pack != 0, cus);
+}
 """
 
 
@@ -43,3 +46,17 @@ def test_other_shapes_stay_on_the_tile_kernel(rules):
     for m, n, f16 in [(64, 80, 0), (128, 144, 1), (86, 128, 1), (108, 128, 0), (76, 128, 1), (96, 96, 1), (112, 64, 1)]:
         for tokens in (1, 256, 300, 512, 600, 1024, 4096):
             assert not rules.padded_mfma(m, n, ctypes.c_int64(tokens), f16, ctypes.c_int64(CUS)), (m, n, f16, tokens)
+
+
+def test_few_features_and_tokens_on_the_generic_kernel(rules):
+    def takes(m, n, tokens, f32, pack):
+        return bool(rules.generic_few(m, n, ctypes.c_int64(tokens), int(f32), int(pack), ctypes.c_int64(CUS)))
+
+    for tokens in (1, 255):
+        assert takes(8, 8, tokens, False, False) and takes(8, 12, tokens, True, False) and takes(4, 4, tokens, True, True)
+        assert takes(4, 6, tokens, True, False)
+        assert not takes(8, 12, tokens, False, False) and not takes(12, 12, tokens, True, False)
+        assert not takes(5, 8, tokens, False, False) and not takes(8, 8, tokens, False, True) and not takes(4, 8, tokens, True, True)
+    for f32 in (False, True):
+        for pack in (False, True):
+            assert not takes(4, 4, 256, f32, pack) and not takes(64, 64, 1, f32, pack)
