@@ -42,4 +42,26 @@ inline bool fq_generic_few(int M, int N, int64_t tokens, bool f32, bool pack, in
   return f32 && F <= 32;
 }
 
+// Ragged products (N % 4 != 0 or K % 128 != 0) that the generic GEMM kernel
+// finishes sooner than the small-M kernel (`over_skinny`) or the FP6 route. A
+// workgroup of the generic kernel makes 16 x 16 outputs; two per CU run beside
+// each other, further rounds of them cost more (in ns, per k: 20 for the first
+// round on W.t(), 25 on [K/8, N], 26 for each further one). The small-M kernel
+// takes 3.7 to 5 us whatever K is here, the FP6 route's two launches 6 to 9 us
+// of the device and 9.3 us of the host (one launch: 5.8 us), so the line lies
+// where the generic kernel's estimate passes the device's time but not yet the
+// host's (8 us; single shapes there differ by 2 us either way). Measured on W.t(),
+// FP6 route -> generic: 300 x 64 x 8 6.6 -> 2.4 us, 256 x 37 x 64 7.0 -> 3.5 us,
+// 128 x 1001 x 200 7.9 -> 7.1 us, 128 x 513 x 264 8.8 -> 8.1 us, 256 x 1001 x 64
+// (two rounds) 7.7 -> 6.4 us, but 512 x 1001 x 64 (four) 8.1 against 10.5 and
+// 65 x 1001 x 320 7.5 against 9.1; [K/8, N] 65 x 1001 x 264 7.6 against 9.0.
+// Small-M kernel -> generic: 64 x 37 x 64 4.3 -> 3.5 us, 64 x 2051 x 32 4.7 -> 3.4
+// us, 16 x 513 x 96 4.0 either way.
+inline bool gemm_generic_small(int64_t M, int64_t N, int64_t K, bool b_nk, bool over_skinny, int64_t cus) {
+  const int64_t blocks = ((M + 15) / 16) * ((N + 15) / 16);
+  const int64_t rounds = (blocks + 2 * cus - 1) / (2 * cus);
+  if (over_skinny) return K * rounds <= 64;
+  return 2000 + K * ((b_nk ? 20 : 25) + 26 * (rounds - 1)) <= 8000;
+}
+
 }  // namespace qo

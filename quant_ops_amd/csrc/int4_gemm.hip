@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "dispatch_rules.h"
 #include "int4_common.h"
 
 #ifndef QO_GEMM_TILE
@@ -1398,36 +1399,63 @@ static bool f6_route(int64_t M, int64_t N, int64_t K, int out_dtype, int64_t bsp
          (bsp == 1 || bsn == 1) && !route_off(QO_ROUTE_GEMM_NO_F6);
 }
 
+// What a call's dispatch needs to know of its operands.
+struct GemmOperands {
+  bool b_nk, b_kn;       // B is the W.t() view / row-major
+  bool fits;             // 32-bit in-tile byte offsets of the pipelined kernels: 256 rows of A or B
+  bool aligned_in;       // 16-byte rows of A and B
+  bool aligned;          // and output rows of 4-element groups
+  bool dma_layout;       // the small-M kernel's LDS-DMA form takes B
+  int64_t ldb;
+};
+static GemmOperands gemm_operands(const void* a, int64_t lda, const void* b, int64_t bsp, int64_t bsn, const void* out,
+                                  int64_t out_size, int64_t ldc, int64_t M, int64_t N, int64_t K) {
+  GemmOperands o;
+  o.b_nk = bsp == 1;
+  o.b_kn = bsn == 1 && !o.b_nk;
+  o.ldb = o.b_nk ? bsn : bsp;
+  o.fits = M <= INT32_MAX / 2 && N <= INT32_MAX / 2 && K <= 65536 && lda < (1 << 21) && o.ldb < (1 << 21);
+  o.aligned_in = (uintptr_t)a % 16 == 0 && lda % 4 == 0 && (uintptr_t)b % 16 == 0 && o.ldb % 4 == 0;
+  o.aligned = o.aligned_in && (uintptr_t)out % (4 * out_size) == 0 && ldc % 4 == 0;
+  o.dma_layout = o.b_nk || skinny_kn_dma_ok(N, K, o.ldb);
+  return o;
+}
+
+// The first choice of a call: the small-M kernel, the FP6 route (which needs a
+// workspace), the generic kernel for small ragged products, or the kernels
+// chosen further down.
+enum class GemmRoute { kSkinny, kF6, kSmall, kRest };
+static GemmRoute gemm_route(const GemmOperands& o, int64_t M, int64_t N, int64_t K, int out_dtype, int64_t bsp,
+                            int64_t bsn) {
+  // decode shapes: the skinny kernel (columns x K-slices, B streamed once); the
+  // LDS-DMA form also takes rows of whole 16-byte pieces that end inside a stage
+  const bool skinny = o.fits && o.aligned_in && (o.b_nk || o.b_kn) && M <= 64 && K > 0 && gemm_allow_skinny() &&
+                      (K % 128 == 0 || (K % 32 == 0 && o.dma_layout)) && (o.b_nk || o.dma_layout || o.aligned);
+  if (ragged(N, K) && gemm_generic_small(M, N, K, o.b_nk, skinny, device_cu_count())) return GemmRoute::kSmall;
+  if (skinny) return GemmRoute::kSkinny;
+  return f6_route(M, N, K, out_dtype, bsp, bsn) ? GemmRoute::kF6 : GemmRoute::kRest;
+}
+
 template <class OT>
 static void dispatch(const int32_t* a, int64_t lda, const int32_t* b, int64_t bsp, int64_t bsn, const void* sa,
                      int sad, const void* sb, int sbd, void* out, int64_t ldc, const void* bias, int64_t M, int64_t N, int64_t K,
                      hipStream_t stream, bool allow_fast, void* workspace, int64_t ws_bytes) {
   using T = typename OT::T;
   constexpr int kOut = std::is_same_v<OT, OutF16> ? QO_DTYPE_F16 : std::is_same_v<OT, OutBF16> ? QO_DTYPE_BF16 : QO_DTYPE_F32;
-  const bool f6 = allow_fast && workspace && (uintptr_t)workspace % 256 == 0 && f6_route(M, N, K, kOut, bsp, bsn) &&
-                  ws_bytes >= f6_workspace_bytes(M, N, K);
-  const bool b_nk = (bsp == 1);
-  const bool b_kn = (bsn == 1) && !b_nk;
-  const int64_t ldb = b_nk ? bsn : bsp;
-  // 32-bit in-tile byte offsets of the pipelined kernels: 256 rows of A or B
-  const bool fits = M <= INT32_MAX / 2 && N <= INT32_MAX / 2 && K <= 65536 && lda < (1 << 21) &&
-                    ldb < (1 << 21);
-  const bool aligned_in = ((uintptr_t)a % 16 == 0) && (lda % 4 == 0) && ((uintptr_t)b % 16 == 0) && (ldb % 4 == 0);
-  const bool aligned = aligned_in && ((uintptr_t)out % (4 * sizeof(T)) == 0) && (ldc % 4 == 0);
-  const bool dma_layout = b_nk || skinny_kn_dma_ok(N, K, ldb);
-  // decode shapes: the skinny kernel (columns x K-slices, B streamed once); the
-  // LDS-DMA form also takes rows of whole 16-byte pieces that end inside a stage
-  if (allow_fast && fits && aligned_in && (b_nk || b_kn) && M <= 64 && K > 0 && gemm_allow_skinny() &&
-      (K % 128 == 0 || (K % 32 == 0 && dma_layout)) && (b_nk || dma_layout || aligned)) {
+  const GemmOperands o = gemm_operands(a, lda, b, bsp, bsn, out, sizeof(T), ldc, M, N, K);
+  const GemmRoute route = allow_fast ? gemm_route(o, M, N, K, kOut, bsp, bsn) : GemmRoute::kSmall;
+  const bool b_nk = o.b_nk, dma_layout = o.dma_layout;
+  const int64_t ldb = o.ldb;
+  if (route == GemmRoute::kSkinny) {
     launch_skinny<OT>(a, lda, b, ldb, b_nk, sa, sad, sb, sbd, out, ldc, bias, (int)M, (int)N, (int)K, stream);
     return;
   }
-  if (f6) {
+  if (route == GemmRoute::kF6 && workspace && (uintptr_t)workspace % 256 == 0 && ws_bytes >= f6_workspace_bytes(M, N, K)) {
     f6_gemm_launch<OT>(a, lda, b, bsp, bsn, sa, sad, sb, sbd, static_cast<T*>(out), ldc, static_cast<const T*>(bias),
                        M, N, K, workspace, stream);
     return;
   }
-  if (allow_fast && fits && aligned && (b_nk || b_kn)) {
+  if (route != GemmRoute::kSmall && o.fits && o.aligned && (b_nk || o.b_kn)) {
     const int m = (int)M, n = (int)N, k = (int)K;
     // Up to 256 rows over few columns (the tiled grid would fill at most 1/8
     // of the CUs, each tile streaming all of K): one skinny launch per 128

@@ -14,6 +14,9 @@ SOURCE = r"""
 extern "C" int padded_mfma(int M, int N, int64_t tokens, int f16, int64_t cus) {
   return qo::fq_padded_mfma(M, N, tokens, f16 != 0, cus);
 }
+extern "C" int generic_small(int64_t M, int64_t N, int64_t K, int b_nk, int over_skinny, int64_t cus) {
+  return qo::gemm_generic_small(M, N, K, b_nk != 0, over_skinny != 0, cus);
+}
 extern "C" int generic_few(int M, int N, int64_t tokens, int f32, int pack, int64_t cus) {
   return qo::fq_generic_few(M, N, tokens, f32 != 0, pack != 0, cus);
 }
@@ -60,3 +63,19 @@ def test_few_features_and_tokens_on_the_generic_kernel(rules):
     for f32 in (False, True):
         for pack in (False, True):
             assert not takes(4, 4, 256, f32, pack) and not takes(64, 64, 1, f32, pack)
+
+
+def test_small_ragged_products_on_the_generic_kernel(rules):
+    def takes(m, n, k, over_skinny, b_nk=True):
+        return bool(rules.generic_small(*(ctypes.c_int64(v) for v in (m, n, k)), int(b_nk), int(over_skinny),
+                                        ctypes.c_int64(CUS)))
+
+    for m, n, k in [(1, 64, 8), (1024, 64, 8), (256, 37, 64), (300, 64, 200), (128, 1001, 200), (256, 1001, 64), (1, 1, 64)]:
+        assert takes(m, n, k, False) and takes(m, n, k, False, b_nk=False), (m, n, k)
+    assert takes(128, 513, 264, False) and not takes(128, 513, 264, False, b_nk=False)
+    for m, n, k in [(512, 1001, 64), (256, 1001, 200), (1, 5, 328), (1, 1, 4096), (16, 1631, 8064), (4096, 4095, 64)]:
+        assert not takes(m, n, k, False) and not takes(m, n, k, False, b_nk=False), (m, n, k)
+    for m, n, k in [(1, 5, 32), (64, 37, 64), (64, 2051, 32)]:
+        assert takes(m, n, k, True), (m, n, k)
+    for m, n, k in [(1, 5, 96), (64, 2051, 64), (16, 151643, 4096), (64, 4095, 64)]:
+        assert not takes(m, n, k, True), (m, n, k)

@@ -41,3 +41,23 @@ def test_padded_shapes_at_their_lines(gpu, m, n, tokens, dtype, pack, routing):
     assert same.float().mean() >= 0.97
     d = (_codes(q, pack) - _codes(qg, pack)).abs()[same]
     assert int(d.max()) <= 1 and (d > 0).float().mean().item() <= 1e-3
+
+
+@pytest.mark.parametrize("w_view", [True, False])
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m", [1, 16, 17, 64, 65, 128, 300])
+@pytest.mark.parametrize("n,k", [(5, 64), (5, 160), (37, 192), (2051, 32), (2052, 64), (1023, 288), (64, 200), (64, 264), (1001, 72)])
+def test_ragged_gemm_at_the_lines(gpu, m, n, k, out_dtype, w_view, routing):
+    """Small ragged products (generic kernel) and the next larger ones (small-M kernel with 1 to 3 lane groups in
+    the last stage, FP6 route): the sums are exact on all of them, so outputs are equal bit for bit."""
+    print(f"[gpu-dispatch] {m}x{n}x{k} {out_dtype} W.t()={w_view}", flush=True)
+    case = wl.gemm_case(m, n, k, seed=m + n + k, b_transposed_view=w_view, out_dtype=out_dtype)
+    a, b, sa, sb = case.a.to(gpu), case.b.to(gpu), case.scale_a.to(gpu).float(), case.scale_b.to(gpu)
+    wide = torch.full((m, n + 5), 7.0, dtype=out_dtype, device=gpu)   # rows at a stride above their length
+    out = wide[:, :n]
+    capi.int4_gemm(a, b, sa, sb, out_dtype=out_dtype, out=out, workspace=True)
+    routing.on("GEMM_GENERIC")
+    ref = capi.int4_gemm(a, b, sa, sb, out_dtype=out_dtype)
+    routing.off("GEMM_GENERIC")
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref) and bool((wide[:, n:] == 7.0).all())
