@@ -161,9 +161,10 @@ int qo_int4_gemm_bias(const int32_t* a, int64_t lda,
  *   workspace        device memory, 256-byte aligned, workspace_bytes long;
  *                    only read and written by this call's kernels on stream
  *                    (calls sharing a workspace must be ordered)
- *   workspace_bytes  at least qo_int4_gemm_workspace_size(M, N, K, out_dtype)
- *                    for the FP6 route; a smaller (or NULL) workspace takes
- *                    qo_int4_gemm's kernels
+ *   workspace_bytes  at least qo_int4_gemm_workspace_needed(...) of the same
+ *                    operands (or qo_int4_gemm_workspace_size(M, N, K,
+ *                    out_dtype), which is never less) for the FP6 route; a
+ *                    smaller (or NULL) workspace takes qo_int4_gemm's kernels
  *
  * Errors: those of qo_int4_gemm.
  */
@@ -177,8 +178,20 @@ int qo_int4_gemm_ws(const int32_t* a, int64_t lda,
                     void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
- * Workspace bytes qo_int4_gemm_ws uses for an M x N x K product with outputs
- * of out_dtype: 0 when the shape does not take the FP6 route (M <= 256 or float32
+ * Workspace bytes that qo_int4_gemm_ws uses for exactly these operands (same
+ * arguments as there; nothing is read through the pointers, only their
+ * alignment counts): 0 where the call takes a kernel without a workspace, for
+ * instance the small-M kernel at up to 64 rows of a ragged W.t(), else
+ * qo_int4_gemm_workspace_size.
+ */
+int64_t qo_int4_gemm_workspace_needed(const int32_t* a, int64_t lda,
+                                      const int32_t* b, int64_t b_stride_p, int64_t b_stride_n,
+                                      const void* out, int out_dtype, int64_t ldc,
+                                      int64_t M, int64_t N, int64_t K);
+
+/*
+ * The most workspace bytes qo_int4_gemm_ws uses for an M x N x K product with
+ * outputs of out_dtype, whatever B's layout and the operands' alignment: 0 when the shape does not take the FP6 route (M <= 256 or float32
  * outputs where N % 4 == 0 and K % 128 == 0, K > 65536, or QO_ROUTE_GEMM_NO_F6 or
  * QO_ROUTE_GEMM_GENERIC set), else
  * qo_int4_gemm_f6_workspace_bytes(M, N, K): 0.75 (M + N) K bytes plus padding

@@ -20,7 +20,7 @@ STATUS = {0: "QO_OK", 1: "QO_ERR_NULL_POINTER", 2: "QO_ERR_SHAPE", 3: "QO_ERR_DT
 
 # Every symbol the header declares; the CPU tests check they are all exported.
 EXPORTED = ("qo_status_string", "qo_version", "qo_last_error", "qo_set_kernel_routing", "qo_flatquant_quantize",
-            "qo_int4_gemm", "qo_int4_gemm_bias", "qo_int4_gemm_ws", "qo_int4_gemm_workspace_size", "qo_int4_gemm_f6_workspace_bytes",
+            "qo_int4_gemm", "qo_int4_gemm_bias", "qo_int4_gemm_ws", "qo_int4_gemm_workspace_size", "qo_int4_gemm_workspace_needed", "qo_int4_gemm_f6_workspace_bytes",
             "qo_int4_gemm_f6_prepare", "qo_int4_gemm_f6_run", "qo_int4_gemm_f6_operand_bytes",
             "qo_int4_gemm_f6_convert", "qo_int4_gemm_f6_run2", "qo_w4a4_linear_f6w", "qo_w4a4_linear", "qo_w4a4_linear_ws", "qo_w4a4_linear_noalloc", "qo_dequantize_int4",
             "qo_pack_int4_to_int32", "qo_pack_int4_clamped", "qo_unpack_int32_to_int4", "qo_transpose_int32")
@@ -73,6 +73,8 @@ def lib():
                                   c_i64, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp]
     L.qo_int4_gemm_workspace_size.restype = c_i64
     L.qo_int4_gemm_workspace_size.argtypes = [c_i64, c_i64, c_i64, c_int]
+    L.qo_int4_gemm_workspace_needed.restype = c_i64
+    L.qo_int4_gemm_workspace_needed.argtypes = [c_vp, c_i64, c_vp, c_i64, c_i64, c_vp, c_int, c_i64, c_i64, c_i64, c_i64]
     L.qo_int4_gemm_f6_workspace_bytes.restype = c_i64
     L.qo_int4_gemm_f6_workspace_bytes.argtypes = [c_i64, c_i64, c_i64]
     L.qo_int4_gemm_f6_prepare.restype = c_int
@@ -175,7 +177,8 @@ def flatquant_quantize(x, left, right, clip_ratio=1.0, pack_int32=False, out_cod
 
 
 def gemm_workspace_size(m, n, k, out_dtype=torch.float16):
-    """``qo_int4_gemm_workspace_size``: bytes of the FP6 route's workspace (0: not taken)."""
+    """``qo_int4_gemm_workspace_size``: bytes of the FP6 route's workspace, whatever the operands' layout
+    (0: not taken)."""
     return int(lib().qo_int4_gemm_workspace_size(m, n, k, _TORCH_CODE[out_dtype]))
 
 

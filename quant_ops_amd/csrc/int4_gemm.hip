@@ -1577,6 +1577,16 @@ extern "C" int qo_int4_gemm_ws(const int32_t* a, int64_t lda, const int32_t* b, 
                     scale_b_dtype, out, out_dtype, ldc, bias, M, N, K, stream, workspace, workspace_bytes);
 }
 
+extern "C" int64_t qo_int4_gemm_workspace_needed(const int32_t* a, int64_t lda, const int32_t* b, int64_t b_stride_p,
+                                                 int64_t b_stride_n, const void* out, int out_dtype, int64_t ldc,
+                                                 int64_t M, int64_t N, int64_t K) {
+  using namespace qo;
+  if (!gemm_allow_fast() || !is_float_code(out_dtype) || M < 1 || N < 1 || K < 8 || K % 8 != 0) return 0;
+  const GemmOperands o =
+      gemm_operands(a, lda, b, b_stride_p, b_stride_n, out, out_dtype == QO_DTYPE_F32 ? 4 : 2, ldc, M, N, K);
+  return gemm_route(o, M, N, K, out_dtype, b_stride_p, b_stride_n) == GemmRoute::kF6 ? f6_workspace_bytes(M, N, K) : 0;
+}
+
 extern "C" int64_t qo_int4_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int out_dtype) {
   // sized for either B layout (the route also needs one unit stride of B)
   if (!gemm_allow_fast() || K % 8 != 0 || !qo::f6_route(M, N, K, out_dtype, 1, 0)) return 0;

@@ -115,9 +115,10 @@ at::Tensor int4_matmul_impl(const at::Tensor& a, const at::Tensor& b, const at::
     // the reference adds bias.to(output dtype) to the output
     bv = bias->to(out_dtype).contiguous();
   }
-  // workspace of the FP6 route for the large shapes (the caching allocator's
+  // workspace of the FP6 route where this call takes it (the caching allocator's
   // blocks are 512-byte aligned)
-  const int64_t ws_bytes = qo_int4_gemm_workspace_size(M, N, K, od);
+  const int64_t ws_bytes = qo_int4_gemm_workspace_needed(A.data_ptr<int32_t>(), lda, B.data_ptr<int32_t>(), bsp, bsn,
+                                                         out.data_ptr(), od, N, M, N, K);
   at::Tensor ws = ws_bytes > 0 ? at::empty({ws_bytes}, a.options().dtype(at::kByte)) : at::Tensor();
   check_status(qo_int4_gemm_ws(A.data_ptr<int32_t>(), lda, B.data_ptr<int32_t>(), bsp, bsn, sa.data_ptr(), sad,
                                sb.data_ptr(), sbd, bv.defined() ? bv.data_ptr() : nullptr, out.data_ptr(), od, N, M,
@@ -185,8 +186,10 @@ at::Tensor w4a4_linear(const at::Tensor& x, const at::Tensor& left_trans, const 
   at::Tensor codes = at::empty({T, F / 8}, x.options().dtype(at::kInt));
   at::Tensor scales = at::empty({T}, x.options().dtype(at::kFloat));
   at::Tensor out = at::empty({T, NO}, x.options());
-  // the GEMM's FP6 route at large token counts (0 bytes: not taken)
-  const int64_t ws_bytes = qo_int4_gemm_workspace_size(T, NO, F, code);
+  // the GEMM's FP6 route (0 bytes: not taken)
+  const int64_t ws_bytes =
+      qo_int4_gemm_workspace_needed(codes.data_ptr<int32_t>(), F / 8, W.data_ptr<int32_t>(), 1,
+                                    NO > 0 ? W.stride(0) : F / 8, out.data_ptr(), code, NO, T, NO, F);
   at::Tensor ws = ws_bytes > 0 ? at::empty({ws_bytes}, x.options().dtype(at::kByte)) : at::Tensor();
   check_status(qo_w4a4_linear_ws(X.data_ptr(), code, T, T > 0 ? X.stride(0) : F, L.data_ptr(), R.data_ptr(), (int)M,
                                  (int)N, (float)clip_ratio, W.data_ptr<int32_t>(), NO > 0 ? W.stride(0) : F / 8, NO,

@@ -358,3 +358,31 @@ def test_kernel_routing_mask_round_trips():
         assert capi.set_kernel_routing(0) == 0
     finally:
         capi.set_kernel_routing(prev)
+
+
+def test_gemm_workspace_of_a_call_without_gpu():
+    """qo_int4_gemm_workspace_needed looks at layout and alignment, not only at the sizes."""
+    need = capi.lib().qo_int4_gemm_workspace_needed
+
+    def call(m, n, k, w_view, out_dtype=1, a=4096, out=4096, ldc=None):
+        kp = k // 8
+        strides = (1, kp) if w_view else (n, 1)
+        return need(a, kp, 8192, *strides, out, out_dtype, ldc or n, m, n, k)
+
+    # the small-M kernel: up to 64 rows of whole 16-byte pieces
+    for m in (1, 16, 64):
+        assert call(m, 151643, 4096, True) == 0 and call(m, 1631, 8064, True) == 0 and call(m, 1632, 8128, False) == 0
+    # not in its reach: an odd N of [K/8, N], rows that are no whole pieces, unaligned A, more rows
+    for args in ((16, 1631, 8064, False), (16, 1631, 8072, True), (65, 151643, 4096, True)):
+        assert call(*args) == capi.gemm_workspace_size(*args[:3]) > 0
+    assert call(16, 1631, 8064, True, a=4100) > 0
+    # small ragged products: the generic kernel
+    assert call(300, 64, 8, True) == 0 and call(1, 5, 32, False) == 0
+    # large products as before, and never more than the size for any layout
+    assert call(257, 4096, 4096, True) == call(257, 4096, 4096, False) == capi.gemm_workspace_size(257, 4096, 4096) > 0
+    assert call(256, 4096, 4096, True) == 0 and call(4096, 4096, 4096, True, out_dtype=0) == 0
+    assert call(0, 4096, 4096, True) == 0 and call(300, 4096, 4100, True) == 0 and call(300, 4096, 4096, True, out_dtype=9) == 0
+    with capi.kernel_routing("GEMM_NO_F6"):
+        assert call(4096, 4096, 4096, True) == 0
+    with capi.kernel_routing("GEMM_NO_SKINNY"):
+        assert call(16, 1631, 8064, True) > 0
