@@ -38,6 +38,18 @@ void* current_stream(const at::Tensor& t) {
   return reinterpret_cast<void*>(c10::hip::getCurrentHIPStream(t.device().index()).stream());
 }
 
+// The FP6 route's workspace from the caching allocator (its blocks are 512-byte
+// aligned); undefined where no byte is needed, or where memory does not allow
+// it: the GEMM then takes the kernels that need none, with the same results.
+at::Tensor gemm_workspace(int64_t bytes, const at::Tensor& like) {
+  if (bytes <= 0) return at::Tensor();
+  try {
+    return at::empty({bytes}, like.options().dtype(at::kByte));
+  } catch (const c10::OutOfMemoryError&) {
+    return at::Tensor();
+  }
+}
+
 // Same checks as cuda_kronecker_quant_int8 (cuda_quant_kernel.cu:324-329), plus
 // the dtype agreement torch::matmul enforces there.
 std::tuple<at::Tensor, at::Tensor> flatquant_dynamic_quantize(const at::Tensor& input, const at::Tensor& left_trans,
@@ -115,11 +127,9 @@ at::Tensor int4_matmul_impl(const at::Tensor& a, const at::Tensor& b, const at::
     // the reference adds bias.to(output dtype) to the output
     bv = bias->to(out_dtype).contiguous();
   }
-  // workspace of the FP6 route where this call takes it (the caching allocator's
-  // blocks are 512-byte aligned)
   const int64_t ws_bytes = qo_int4_gemm_workspace_needed(A.data_ptr<int32_t>(), lda, B.data_ptr<int32_t>(), bsp, bsn,
                                                          out.data_ptr(), od, N, M, N, K);
-  at::Tensor ws = ws_bytes > 0 ? at::empty({ws_bytes}, a.options().dtype(at::kByte)) : at::Tensor();
+  at::Tensor ws = gemm_workspace(ws_bytes, a);
   check_status(qo_int4_gemm_ws(A.data_ptr<int32_t>(), lda, B.data_ptr<int32_t>(), bsp, bsn, sa.data_ptr(), sad,
                                sb.data_ptr(), sbd, bv.defined() ? bv.data_ptr() : nullptr, out.data_ptr(), od, N, M,
                                N, K, ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(a)),
@@ -190,7 +200,7 @@ at::Tensor w4a4_linear(const at::Tensor& x, const at::Tensor& left_trans, const 
   const int64_t ws_bytes =
       qo_int4_gemm_workspace_needed(codes.data_ptr<int32_t>(), F / 8, W.data_ptr<int32_t>(), 1,
                                     NO > 0 ? W.stride(0) : F / 8, out.data_ptr(), code, NO, T, NO, F);
-  at::Tensor ws = ws_bytes > 0 ? at::empty({ws_bytes}, x.options().dtype(at::kByte)) : at::Tensor();
+  at::Tensor ws = gemm_workspace(ws_bytes, x);
   check_status(qo_w4a4_linear_ws(X.data_ptr(), code, T, T > 0 ? X.stride(0) : F, L.data_ptr(), R.data_ptr(), (int)M,
                                  (int)N, (float)clip_ratio, W.data_ptr<int32_t>(), NO > 0 ? W.stride(0) : F / 8, NO,
                                  sw.data_ptr(), swd, bv.defined() ? bv.data_ptr() : nullptr,

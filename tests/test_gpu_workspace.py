@@ -36,3 +36,24 @@ def test_decode_over_an_odd_vocabulary_takes_no_workspace(gpu, m):
     _, peak = _peak(lambda: torch.ops.quant_ops.w4a4_linear(x, left, right, b.t(), sb, 0.9, None))
     print(f"[gpu-workspace] w4a4_linear {m}x{n}x{k}: {peak} bytes", flush=True)
     assert peak < ROOM
+
+
+@pytest.mark.parametrize("m,w_view", [(16, False), (200, True), (300, True)])
+def test_gemm_without_room_for_its_workspace(gpu, m, w_view):
+    """Where the caching allocator cannot give the FP6 route's workspace (here: its share of the memory is
+    capped from the host), the call takes the kernels without one and gives the same output."""
+    n, k = 40001, 4096
+    case = wl.gemm_case(m, n, k, seed=m, b_transposed_view=w_view)
+    a, b, sa, sb = case.a.to(gpu), case.b.to(gpu), case.scale_a.to(gpu), case.scale_b.to(gpu)
+    full, peak = _peak(lambda: qo.int4_matmul(a, b, sa, sb))
+    ws = capi.gemm_workspace_size(m, n, k)
+    assert peak > ws > (100 << 20)   # the FP6 route
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + ws // 2) / total)
+    try:
+        out, peak = _peak(lambda: qo.int4_matmul(a, b, sa, sb))
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    print(f"[gpu-workspace] {m}x{n}x{k} capped: {peak} bytes", flush=True)
+    assert peak < ws and torch.equal(out, full)
