@@ -36,6 +36,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "dispatch_rules.h"
 #include "int4_common.h"
 
 namespace qo {
@@ -663,42 +664,6 @@ int64_t f6_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return align256(f6_operand_bytes(M, K)) + f6_operand_bytes(N, K);
 }
 
-namespace {
-// The output tile of an M x N x K product, by an estimate of its time in ns: k-blocks
-// times the time of a round's stages, plus what a round takes besides them. A
-// stage is bound by the CU's LDS traffic (its operand reads at about 128 bytes
-// per clock, the copies from L2 at 64), so a larger tile costs less per product
-// but leaves more CUs idle. Per stage, measured at 4096 columns x 14336: 256-row
-// tiles 740 (850 with every CU busy, 256 columns wide), 128 x 128 430 for one
-// workgroup on a CU and 700 for two, 128 x 64 345 and 480; per round 8 us and 4 us.
-// Split tiles (one per CU, two groups of waves) take 670 and 510 for a pair of
-// stages, and 1 us more a round for the sums' exchange: they win where a round
-// leaves CUs with one tile and K is 1536 or more. Kernel alone, unsplit -> split:
-// 512 x 4096 x 14336 38.6 -> 33.8 us, 640 x 3584 x 18944 61.1 -> 49.2 us,
-// 400 x 8192 x 28672 94.6 -> 80.2 us, 1024 x 4096 x 14336 49.7 -> 42.1 us,
-// 300 x 2048 x 2048 7.7 -> 7.4 us.
-// With 256-row tiles alone M = 512 took 83.7 us there (38 tiles on 256 CUs), on
-// 128 x 64 it takes 40 us; 512 x 14336 x 4096 33 -> 25 us on 128 x 128; 2048 x
-// 4096 x 4096 34 -> 25 us; 2048 x 14336 x 4096 keeps 256 x 224 (87 us against 94).
-enum F6Tile { kF6Tile224, kF6Tile256, kF6Tile128, kF6Tile64, kF6Split128, kF6Split64 };
-F6Tile f6_tile(int64_t M, int64_t N, int64_t K, bool f32) {
-  const int64_t cus = device_cu_count(), nk = (K + 127) / 128;
-  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  auto wide = [&](int64_t t, int64_t stage) { return (t + cus - 1) / cus * (nk * stage + 8000); };
-  auto pair = [&](int64_t t, int64_t one, int64_t two) {   // rounds of two workgroups per CU
-    const int64_t full = t / (2 * cus), rest = t % (2 * cus);
-    return full * (nk * two + 4000) + (rest == 0 ? 0 : nk * (rest <= cus ? one : two) + 4000);
-  };
-  auto split = [&](int64_t t, int64_t stage) { return (t + cus - 1) / cus * ((nk + 1) / 2 * stage + 5000); };
-  const int64_t est[6] = {wide(tiles(256, 224), 745), wide(tiles(256, 256), 850), pair(tiles(128, 128), 430, 700),
-                          pair(tiles(128, 64), 345, 480), split(tiles(128, 128), 670), split(tiles(128, 64), 510)};
-  int best = f32 ? 2 : 0;   // the 256-row kernel stages 16-bit values
-  for (int i = best + 1; i < 6; ++i)
-    if (est[i] < est[best]) best = i;
-  return (F6Tile)best;
-}
-}  // namespace
-
 void f6_prepare(const int32_t* a, int64_t lda, const int32_t* b, int64_t bsp, int64_t bsn, int64_t M, int64_t N,
                 int64_t K, void* workspace, hipStream_t stream) {
   uint8_t* a6 = static_cast<uint8_t*>(workspace);
@@ -734,7 +699,7 @@ void f6_run2(const void* a6v, const void* b6v, const void* sa, int sad, const vo
            (int)((N + 31) / 32), (int)((K + 127) / 128), sa, sad, sb, sbd, out, ldc, bias, (int)M, (int)N, tiles_m);
   };
   constexpr bool kF32 = std::is_same_v<OT, OutF32>;
-  switch (f6_tile(M, N, K, kF32)) {
+  switch (f6_tile(M, N, K, kF32, device_cu_count())) {
     case kF6Tile224:
       if constexpr (!kF32) go(gemm_f6_pp2<256, 224, OT>, 256, 224, 512);
       break;

@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+from test_gpu_f6_tiles import CASES, SPLIT_CASES
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CUS = 256
 
@@ -17,6 +19,7 @@ extern "C" int padded_mfma(int M, int N, int64_t tokens, int f16, int64_t cus) {
 extern "C" int generic_small(int64_t M, int64_t N, int64_t K, int b_nk, int over_skinny, int64_t cus) {
   return qo::gemm_generic_small(M, N, K, b_nk != 0, over_skinny != 0, cus);
 }
+extern "C" int tile(int64_t M, int64_t N, int64_t K, int f32, int64_t cus) { return qo::f6_tile(M, N, K, f32 != 0, cus); }
 extern "C" int generic_few(int M, int N, int64_t tokens, int f32, int pack, int64_t cus) {
   return qo::fq_generic_few(M, N, tokens, f32 != 0, pack != 0, cus);
 }
@@ -79,3 +82,23 @@ def test_small_ragged_products_on_the_generic_kernel(rules):
         assert takes(m, n, k, True), (m, n, k)
     for m, n, k in [(1, 5, 96), (64, 2051, 64), (16, 151643, 4096), (64, 4095, 64)]:
         assert not takes(m, n, k, True), (m, n, k)
+
+
+TILES = ["256x224", "256x256", "128x128", "128x64", "split 128x128", "split 128x64"]   # F6Tile's order
+
+
+@pytest.mark.parametrize("m,n,k,tile,tile_f32", CASES + SPLIT_CASES)
+def test_fp6_tile_of_the_gpu_cases(rules, m, n, k, tile, tile_f32):
+    """The sizes of test_gpu_f6_tiles.py run on the tiles that they are there for."""
+    got = [TILES[rules.tile(*(ctypes.c_int64(v) for v in (m, n, k)), f32, ctypes.c_int64(CUS))] for f32 in (0, 1)]
+    assert got == [tile, tile_f32]
+
+
+def test_fp6_tile_of_common_products(rules):
+    def tile(m, n, k):
+        return TILES[rules.tile(*(ctypes.c_int64(v) for v in (m, n, k)), 0, ctypes.c_int64(CUS))]
+
+    assert tile(4096, 14336, 4096) == "256x224" and tile(2048, 14336, 4096) == "256x224"
+    assert tile(4096, 4096, 14336) == "256x256"
+    assert tile(512, 14336, 4096) == "128x128" and tile(512, 4096, 14336) == "split 128x64"
+    assert tile(400, 8192, 28672) == "split 128x128"

@@ -1,6 +1,7 @@
 """The FP6 GEMM's output tiles at ragged edges, each against the integer route,
 whose sums are exact: outputs are equal bit for bit. The host picks the tile from
-the sizes; which one it is for each case here is in its comment."""
+the sizes (f6_tile, dispatch_rules.h): each case names the one it is meant for,
+and test_dispatch_rules.py checks that on the CPU for 256 CUs."""
 import pytest
 import torch
 
@@ -9,22 +10,32 @@ from quant_ops_amd import workloads as wl
 
 pytestmark = pytest.mark.gpu
 
+# (M, N, K), the tile for 16-bit outputs and for float32 ones
 CASES = [
-    (257, 100, 8),          # 128 x 64, one k-block
-    (300, 333, 136),        # 128 x 64, two
-    (513, 1000, 1000),      # 128 x 64, more k-blocks than the ring has stages
-    (333, 11001, 392),      # 128 x 128, odd N
-    (700, 5003, 1160),      # 128 x 128
-    (1025, 14329, 776),     # 128 x 128, several rounds of workgroups
-    (1000, 14001, 640),     # 256 x 224, odd N
-    (4090, 4099, 2056),     # 256 x 224
-    (4001, 4090, 1032),     # 256 x 256
+    (257, 100, 8, "128x64", "128x64"),          # one k-block
+    (300, 333, 136, "128x64", "128x64"),        # two
+    (513, 1000, 1000, "128x64", "128x64"),      # more k-blocks than the ring has stages
+    (333, 11001, 392, "128x128", "128x128"),    # odd N
+    (700, 5003, 1160, "128x128", "128x128"),
+    (1025, 14329, 776, "128x128", "128x128"),   # several rounds of workgroups
+    (1000, 14001, 640, "256x224", "128x128"),   # odd N
+    (4090, 4099, 2056, "256x224", "128x128"),
+    (4001, 4090, 1032, "256x256", "128x128"),
+]
+SPLIT_CASES = [
+    (300, 333, 2048, "split 128x64", "split 128x64"),     # 16 k-blocks: eight for each group of waves
+    (300, 333, 2056, "split 128x64", "split 128x64"),     # 17: the second group has one less
+    (257, 4097, 2312, "split 128x64", "split 128x64"),    # odd N, 19 k-blocks
+    (300, 11001, 3080, "128x128", "128x128"),             # more tiles than CUs: by one group, 25 k-blocks
+    (300, 10001, 6408, "split 128x128", "split 128x128"), # odd N, 51 k-blocks
+    (511, 4103, 6280, "split 128x128", "split 128x128"),  # 50 k-blocks: 25 for each
+    (511, 4100, 65536, "split 128x128", "split 128x128"), # the largest sums
 ]
 
 
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("m,n,k", CASES)
+@pytest.mark.parametrize("m,n,k", [c[:3] for c in CASES])
 def test_f6_tile_equals_integer_route(gpu, m, n, k, out_dtype, bias):
     print(f"[gpu-f6-tiles] {m}x{n}x{k} {out_dtype} bias={bias}", flush=True)
     case = wl.gemm_case(m, n, k, seed=m + k, b_transposed_view=(m + n) % 2 == 0, out_dtype=out_dtype)
@@ -43,13 +54,7 @@ def test_f6_tile_equals_integer_route(gpu, m, n, k, out_dtype, bias):
 
 
 @pytest.mark.parametrize("out_dtype,bias", [(torch.float16, False), (torch.bfloat16, True), (torch.float32, True)])
-@pytest.mark.parametrize("m,n,k", [
-    (300, 333, 2048),       # 128 x 64 by two groups of waves, 16 k-blocks: eight for each
-    (300, 333, 2056),       # 17: the second group has one less
-    (257, 4097, 2312),      # 128 x 64, odd N, 19 k-blocks
-    (300, 11001, 3080),     # 128 x 128 by two groups, 25 k-blocks
-    (511, 4100, 65536),     # the largest sums
-])
+@pytest.mark.parametrize("m,n,k", [c[:3] for c in SPLIT_CASES])
 def test_f6_split_tile_equals_integer_route(gpu, m, n, k, out_dtype, bias):
     """Tiles whose k-blocks two groups of waves share, against the integer route bit for bit."""
     print(f"[gpu-f6-split] {m}x{n}x{k} {out_dtype} bias={bias}", flush=True)
