@@ -39,6 +39,26 @@ def test_f32_matches_generic_kernel(gpu, m, n, tokens, pack, routing):
     assert torch.equal(s, sg) and torch.equal(q, qg)
 
 
+# the other instances of the kernel's table (rows rounded up to 16 MBX, columns to 64, 128, 192 or 256)
+INSTANCES = [(20, 54), (52, 54), (84, 54), (116, 54), (20, 118), (52, 118), (84, 118), (20, 182), (52, 182), (84, 182),
+             (116, 172), (20, 246), (84, 246), (100, 206)]
+
+
+@pytest.mark.parametrize("m,n,tokens", [(m, n, 300) for m, n in INSTANCES] +
+                         [(17, 24, 1537), (17, 24, 2051), (24, 14, 2049), (24, 30, 5000)])   # three and four tokens per workgroup
+def test_f32_instances_match_generic_kernel(gpu, m, n, tokens, routing):
+    print(f"[gpu-f32] instance {tokens} x {m}x{n}", flush=True)
+    x = wl.activations(tokens, m * n, torch.float32, tokens + m, 0.005, 30.0).to(gpu)
+    left, right = wl.orthogonal(m, m + 1).to(gpu), wl.orthogonal(n, n + 7).to(gpu)
+    for pack in (True, False):
+        q, s = capi.flatquant_quantize(x, left, right, 0.9, pack)
+        routing.on("FQ_GENERIC")
+        qg, sg = capi.flatquant_quantize(x, left, right, 0.9, pack)
+        routing.off("FQ_GENERIC")
+        torch.cuda.synchronize()
+        assert torch.equal(s, sg) and torch.equal(q, qg)
+
+
 @pytest.mark.parametrize("pack", [True, False])
 @pytest.mark.parametrize("m,n,tokens", [(96, 96, 300), (64, 64, 1100), (22, 40, 64)])
 def test_f32_codes_at_ties_bit_exact(gpu, m, n, tokens, pack):

@@ -147,44 +147,44 @@ SHAPES = [
     (4, 32, 32, torch.float16, 1.0, True),
     (7, 64, 32, torch.bfloat16, 0.9, True),
     (5000, 64, 64, torch.float16, 0.9, True),    # more tokens than resident waves: waves loop
-    (11, 16, 16, torch.bfloat16, 1.0, True),     # generic kernel (N not a multiple of 32)
-    (2, 8, 8, torch.float16, 0.9, False),        # generic kernel
-    (5, 12, 20, torch.float32, 1.0, False),      # generic kernel, fp32
+    (11, 16, 16, torch.bfloat16, 1.0, True),     # tile kernel, one block of columns
+    (2, 8, 8, torch.float16, 0.9, False),        # generic kernel (few features and tokens)
+    (5, 12, 20, torch.float32, 1.0, False),      # float32 kernel
     (4, 64, 64, torch.float32, 0.9, True),
     (9, 64, 96, torch.float16, 0.9, True),       # three-wave MFMA groups (N = 96, hidden 6144)
     (5, 80, 128, torch.bfloat16, 1.0, True),     # MFMA kernel, odd M / 16 (hidden 10240)
-    (4, 128, 160, torch.float16, 1.0, False),    # N = 160 (hidden 20480)
-    (2, 128, 192, torch.bfloat16, 0.9, True),    # N = 192 (hidden 24576)
+    (4, 128, 160, torch.float16, 1.0, False),    # tile kernel, N = 160 (hidden 20480)
+    (2, 128, 192, torch.bfloat16, 0.9, True),    # tile kernel, N = 192 (hidden 24576)
     (3, 128, 224, torch.bfloat16, 0.9, True),    # N = 224 (hidden 28672)
-    (6, 64, 80, torch.float16, 0.9, True),       # N zero-padded to 96 (hidden 5120)
+    (6, 64, 80, torch.float16, 0.9, True),       # tile kernel, N zero-padded to 96 (hidden 5120)
     (5, 64, 80, torch.bfloat16, 1.0, False),     # the same, int8 codes
-    (7, 64, 112, torch.bfloat16, 0.9, True),     # N zero-padded to 128 (hidden 7168)
-    (9, 56, 64, torch.float16, 0.9, True),       # M zero-padded to 64 (hidden 3584)
-    (5, 86, 128, torch.bfloat16, 0.9, True),     # M zero-padded to 96, L staged with a partial chunk (11008)
+    (7, 64, 112, torch.bfloat16, 0.9, True),     # tile kernel, N zero-padded to 128 (hidden 7168)
+    (9, 56, 64, torch.float16, 0.9, True),       # tile kernel, M zero-padded to 64 (hidden 3584)
+    (5, 86, 128, torch.bfloat16, 0.9, True),     # tile kernel, M zero-padded to 96, L with a tail (11008)
     (4, 86, 128, torch.float16, 1.0, False),     # the same, int8 codes
-    (6, 108, 128, torch.bfloat16, 1.0, True),    # M zero-padded to 112 (hidden 13824)
-    (3, 128, 144, torch.bfloat16, 0.9, True),    # N zero-padded to 160 (hidden 18432)
+    (6, 108, 128, torch.bfloat16, 1.0, True),    # tile kernel, M zero-padded to 112 (hidden 13824)
+    (3, 128, 144, torch.bfloat16, 0.9, True),    # tile kernel, N zero-padded to 160 (hidden 18432)
     (5, 32, 48, torch.float16, 0.9, True),       # N zero-padded to 64 (hidden 1536)
     (4, 64, 88, torch.bfloat16, 1.0, False),     # N zero-padded to 96 (hidden 5632), int8 codes
-    (6, 80, 112, torch.bfloat16, 0.9, True),     # odd M / 16, N zero-padded to 128 (hidden 8960)
+    (6, 80, 112, torch.bfloat16, 0.9, True),     # tile kernel, odd M / 16, N zero-padded to 128 (hidden 8960)
     (7, 40, 64, torch.float16, 0.9, True),       # M zero-padded to 48 (hidden 2560)
-    (5, 72, 96, torch.bfloat16, 0.9, True),      # M zero-padded to 80, three-wave groups (hidden 6912)
-    (3, 76, 128, torch.float16, 1.0, False),     # M zero-padded to 80 (hidden 9728), int8 codes
-    (5, 128, 148, torch.bfloat16, 0.9, True),    # N = 148 (hidden 18944): rows 8-byte aligned, 16-bit code halves
+    (5, 72, 96, torch.bfloat16, 0.9, True),      # tile kernel, M zero-padded to 80 (hidden 6912)
+    (3, 76, 128, torch.float16, 1.0, False),     # tile kernel, M zero-padded to 80 (hidden 9728), int8 codes
+    (5, 128, 148, torch.bfloat16, 0.9, True),    # tile kernel, N = 148 (hidden 18944): rows in 8-byte pieces
     (4, 128, 148, torch.float16, 1.0, False),    # the same, int8 codes in 4-byte pieces
-    (3, 128, 172, torch.float16, 0.9, True),     # N = 172 (hidden 22016)
-    (1100, 128, 148, torch.float16, 0.9, True),  # 8-byte aligned rows over many tokens
-    (5, 64, 214, torch.bfloat16, 0.9, True),     # N = 214 (hidden 13696): rows 4-byte aligned, byte code stores
+    (3, 128, 172, torch.float16, 0.9, True),     # tile kernel, N = 172 (hidden 22016)
+    (1100, 128, 148, torch.float16, 0.9, True),  # rows in 8-byte pieces over many tokens
+    (5, 64, 214, torch.bfloat16, 0.9, True),     # tile kernel, N = 214 (hidden 13696): rows in 4-byte pieces, byte code stores
     (4, 64, 214, torch.float16, 1.0, False),     # the same, int8 codes in 16-bit pieces
     (2000, 64, 214, torch.float16, 0.9, True),   # the same over many tokens
-    (3, 144, 192, torch.bfloat16, 0.9, True),    # M = 144, odd M / 16 (hidden 27648)
+    (3, 144, 192, torch.bfloat16, 0.9, True),    # tile kernel, M = 144, odd M / 16 (hidden 27648)
     (3, 128, 256, torch.bfloat16, 0.9, True),    # N = 256 (hidden 32768): one X stage
-    (2, 168, 176, torch.float16, 1.0, False),    # both padded, one X stage (hidden 29568), int8 codes
+    (2, 168, 176, torch.float16, 1.0, False),    # tile kernel, both padded (hidden 29568), int8 codes
     (3, 168, 176, torch.bfloat16, 0.9, True),    # the same, packed
     (800, 128, 256, torch.float16, 0.9, True),   # one X stage, groups loop over many tokens
-    (700, 168, 176, torch.bfloat16, 1.0, True),  # the same
-    (4, 160, 160, torch.float16, 1.0, False),    # M = 160 (hidden 25600), int8 codes
-    (900, 160, 160, torch.bfloat16, 0.9, True),  # 160 KB of LDS per group, over many tokens
+    (700, 168, 176, torch.bfloat16, 1.0, True),  # tile kernel over many tokens
+    (4, 160, 160, torch.float16, 1.0, False),    # tile kernel, M = 160 (hidden 25600), int8 codes
+    (900, 160, 160, torch.bfloat16, 0.9, True),  # the same over many tokens
     (3000, 64, 80, torch.bfloat16, 0.9, True),   # padded width, groups loop over many tokens
     (1500, 86, 128, torch.float16, 1.0, True),   # padded height, the same
     (700, 128, 224, torch.bfloat16, 0.9, True),  # L fragments in LDS, the same

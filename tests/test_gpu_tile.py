@@ -91,3 +91,58 @@ def test_tile_codes_at_ties_bit_exact(gpu, m, n, tokens, dtype, pack):
     q, s = capi.flatquant_quantize(x.to(gpu), left.to(gpu), right.to(gpu), 1.0, pack)
     q_ref, s_ref = ofq.flatquant_pytorch(x, left, right, 1.0, pack)
     assert torch.equal(s.cpu(), s_ref.float()) and torch.equal(q.cpu(), q_ref.to(q.dtype))
+
+
+# one shape per instance of the kernel's table (rows rounded up to 16 MBX, columns to 32 KS), widths of 2-element pieces
+_ROWS = {2: 20, 4: 52, 6: 84, 8: 116, 10: 148, 11: 172}
+INSTANCES = [(_ROWS[mbx], 32 * ks - 10) for ks, most in ((1, 4), (2, 6), (3, 8), (4, 10), (5, 11), (6, 11), (7, 11), (8, 11))
+             for mbx in _ROWS if mbx <= most]
+
+
+def _exact(x, left, right, clip):
+    """Codes and scales of the transform in 64 bits throughout."""
+    t, m, n = x.shape[0], left.shape[0], right.shape[0]
+    z = (x.double().reshape(t * m, n) @ right.double()).view(t, m, n)
+    y = (z.transpose(1, 2).reshape(t * n, m) @ left.double()).view(t, n, m).transpose(1, 2).reshape(t, m * n)
+    s = (y.abs().amax(1) * clip / 7.0).clamp(min=1e-8)
+    return torch.round(y / s[:, None]).clamp(-8, 7), s
+
+
+@pytest.mark.parametrize("pack", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n", INSTANCES)
+def test_every_instance_no_further_from_64_bits(gpu, m, n, dtype, pack, routing):
+    """Codes and scales as close to the 64-bit transform as the generic kernel's: the two share every rounding
+    point, so their mean errors differ only by tokens whose sums fall on the other side of a rounding."""
+    print(f"[gpu-tile] instance {m}x{n} {dtype} pack={pack}", flush=True)
+    tokens = 600
+    x = wl.activations(tokens, m * n, dtype, m + n, 0.005, 30.0).to(gpu)
+    left, right = wl.orthogonal(m, m + 1, dtype).to(gpu), wl.orthogonal(n, n + 7, dtype).to(gpu)
+    q, s = capi.flatquant_quantize(x, left, right, 0.9, pack)
+    routing.on("FQ_GENERIC")
+    qg, sg = capi.flatquant_quantize(x, left, right, 0.9, pack)
+    routing.off("FQ_GENERIC")
+    q64, s64 = _exact(x, left, right, 0.9)
+
+    def errors(q, s):
+        return ((s.double() - s64).abs() / s64).mean().item(), (_codes(q, pack) != q64).double().mean().item()
+
+    (se, ce), (sge, cge) = errors(q, s), errors(qg, sg)
+    print(f"[gpu-tile]   scales {se:.3e} (generic {sge:.3e}), codes {ce:.3e} ({cge:.3e})", flush=True)
+    assert se <= 1.02 * sge + 1e-7 and ce <= 1.02 * cge + 1e-6
+    d = (_codes(q, pack) - _codes(qg, pack)).abs()[s == sg]
+    assert (s == sg).float().mean() >= 0.97 and int(d.max()) <= 1 and (d > 0).float().mean().item() <= 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,tokens", [(17, 24, 1537), (17, 24, 2051), (24, 14, 2049), (44, 32, 1790), (24, 30, 5000)])
+def test_several_tokens_per_workgroup(gpu, m, n, tokens, dtype, routing):
+    """Three and four token slots per workgroup, the last group part empty: each token as in a call of its own kind
+    (300 tokens: one slot), bit for bit."""
+    print(f"[gpu-tile] slots {tokens} x {m}x{n} {dtype}", flush=True)
+    x = wl.activations(tokens, m * n, dtype, tokens + m, 0.005, 30.0).to(gpu)
+    left, right = wl.orthogonal(m, m + 1, dtype).to(gpu), wl.orthogonal(n, n + 7, dtype).to(gpu)
+    q, s = capi.flatquant_quantize(x, left, right, 0.9, True)
+    parts = [capi.flatquant_quantize(x[i:i + 300], left, right, 0.9, True) for i in range(0, tokens, 300)]
+    torch.cuda.synchronize()
+    assert torch.equal(q, torch.cat([p[0] for p in parts])) and torch.equal(s, torch.cat([p[1] for p in parts]))
