@@ -72,6 +72,12 @@ __device__ inline uint32_t f32_codes4_div(const v4f& y, float s, bool pack) {
 // Staging of X and of the codes, padding and barriers as in fq_tile_kernel
 // (flatquant_tile.h).
 //
+// R (4 VGPRs per 16-deep slab), X, Z and Y (4 per row block) are all held at
+// once: MBX x KQX = 6 x 12 and 8 x 12 spill 17 and 93 VGPRs, 2, 4, 6 and 8 x 16
+// (128 registers) 17, 87, 148 and 208; every instance spills SGPRs (25 to 83).
+// Those are still 2 times (1024 x 8 x 255) to 9 times (1024 x 64 x 254, 128 x 144)
+// faster than fq_generic_kernel.
+//
 // Bound: the float32 MFMA (64 FLOP per clock and SIMD: a token of 112 x 128 takes
 // a CU 11 us), at small widths the launch and set-up. Measured (kernel alone,
 // before: fq_generic_kernel): 128 x 64 x 64 10.1 -> 7.8 us, 1000 x 64 x 64 32 ->

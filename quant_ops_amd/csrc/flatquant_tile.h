@@ -1,8 +1,11 @@
-// Fused FlatQuant quantize for any even width up to 256 and any height up to
-// 176 (fp16 / bf16): fq_tile_kernel, the kernel behind every shape without one
-// of its own in flatquant_quant.hip. The loops' lengths are compile-time
-// (MBX, KS: the shape rounded up to blocks of 32 rows and columns); M and N
-// themselves are arguments, so 38 instances per type cover every shape.
+// Fused FlatQuant quantize for even widths up to 256 and heights up to 176
+// (fp16 / bf16): fq_tile_kernel, the kernel behind the shapes without one of
+// their own in flatquant_quant.hip. The loops' lengths are compile-time (MBX, KS:
+// the shape rounded up to blocks of 32 rows and columns); M and N themselves are
+// arguments, so 38 instances per type cover every even width and every height
+// but the tall ones: M > 64 with N <= 32, M > 96 with N <= 64, M > 128 with
+// N <= 96 and M > 160 with N <= 128 stay on the generic kernel, as do odd N,
+// N > 256 and M > 176.
 #pragma once
 
 #include <algorithm>
@@ -37,8 +40,13 @@ struct FqTileShape {
   static constexpr int RCH = KS;                  // R
   static constexpr int LCH = (MBX * MBX + 4 * KS - 3) / (4 * KS - 2);   // L
   static constexpr int MAX_THREADS = KS <= 4 ? 512 : 128 * KS;
-  // waves per SIMD the registers are allocated for: what the threads (one
-  // workgroup of 9 to 12 or 13 to 16 waves, or two of up to 8) and the LDS allow
+  // Waves per SIMD the registers are allocated for: what the threads (one
+  // workgroup of 9 to 12 or 13 to 16 waves, or two of up to 8) and the LDS allow.
+  // The price is spilled VGPRs in some instances (fp16, bf16 up to 6 fewer or, at
+  // 10 x 7 and 11 x 7, up to 21): MBX x KS = 8 x 3 13, 8 x 4 17, 10 x 5 and 10 x 6 2
+  // and 6, 11 x 5 and 11 x 6 25 and 29, 6 x 7 and 6 x 8 5 and 7, 8 x 7 and 8 x 8 32
+  // and 38, 10 x 7 and 10 x 8 88 and 72, 11 x 7 and 11 x 8 129; and 14 to 52 SGPRs
+  // (into VGPR lanes) in all of them.
   static constexpr int WAVES_PER_SIMD = KS <= 4 ? (MBX >= 10 ? 2 : 4) : KS <= 6 ? 3 : 4;
 };
 

@@ -169,10 +169,11 @@ __device__ __attribute__((always_inline)) inline void copy_out_c(const unsigned 
   }
 }
 
-// The FP6 route of the tiled GEMM (int4_gemm_f6.hip): workspace bytes for an
+// The FP6 route of the GEMM (int4_gemm_f6.hip): workspace bytes for an
 // M x N x K product, and the two launches (operand conversion into the
-// workspace, then the FP6 GEMM) for 16-bit outputs, M >= 1, N >= 1,
-// K <= 65536 and any strides of A and B.
+// workspace, then the FP6 GEMM) for 16-bit and float32 outputs (the halves
+// below: 16-bit ones), M >= 1, N >= 1, K <= 65536, any row stride of A and one
+// unit stride of B.
 int64_t f6_workspace_bytes(int64_t M, int64_t N, int64_t K);
 template <class OT>
 void f6_gemm_launch(const int32_t* a, int64_t lda, const int32_t* b, int64_t bsp, int64_t bsn, const void* sa,

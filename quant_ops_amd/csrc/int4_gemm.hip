@@ -1337,13 +1337,14 @@ static void launch_skinny(const int32_t* a, int64_t lda, const int32_t* b, int64
     using Cfg = SkinnyNkCfg<MT, false>;
     const int64_t cb = Cfg::CB;
     const bool pair = (K / 2 + cb - 1) / cb <= 2 || (N + 15) / 16 > device_cu_count();
-    if ((NK || kn_dma) && ragged) {
-      if constexpr (MT <= 4)
+    if constexpr (MT <= 4) {   // more rows come here with whole stages and aligned output rows only
+      if ((NK || kn_dma) && ragged) {
         launch((gemm_i4_skinny_nk<MT, false, !NK, OT, true>), grid, dim3(512), 0, stream, a, lda, b, ldb, sa, sad, sb,
                sbd, reinterpret_cast<T*>(out), ldc, reinterpret_cast<const T*>(bias), M, N, K);
-      else if (g_launch_error == hipSuccess)
-        g_launch_error = hipErrorInvalidConfiguration;   // the host sends ragged shapes here up to 64 rows
-    } else if (NK || kn_dma) {
+        return;
+      }
+    }
+    if (NK || kn_dma) {
       bool launched = false;
       if constexpr (Cfg::PAIR_OK) {
         if (pair) {
@@ -1384,14 +1385,15 @@ static void launch_skinny(const int32_t* a, int64_t lda, const int32_t* b, int64
 // generic kernel, a few per cent of the rate.
 static bool ragged(int64_t N, int64_t K) { return N % 4 != 0 || K % 128 != 0; }
 
-// Shapes that take the FP6 route when the caller gives a workspace: the tiled
-// shapes (more than 256 rows; fewer take the small-M kernels) with 16-bit
-// outputs, and ragged ones of any M and output type; B with one unit stride, K
-// within the exact float32 range. Measured against the kernels these ran on
-// before (N x K = 1631 x 8064, bf16 out): 200 rows 641 -> 33 us (W.t()), 16 rows
-// of [K/8, N] 341 -> 30 us; 200 x 1632 x 8128 181 -> 33 us; 315 x 5478 x 11008,
-// float32 out, 4983 -> 60 us. Up to 64 rows of W.t() stay on the small-M kernel
-// (16 x 1631 x 8064 164 -> 6.6 us).
+// Shapes that may take the FP6 route when the caller gives a workspace (calls
+// that the small-M or the generic kernel finishes sooner are taken out before:
+// gemm_route): the tiled shapes (more than 256 rows) with 16-bit outputs, and
+// ragged ones of any M and output type; B with one unit stride, K within the
+// exact float32 range. Measured against the kernels these ran on before (N x K =
+// 1631 x 8064, bf16 out): 200 rows 641 -> 33 us (W.t()), 16 rows of [K/8, N] 341 ->
+// 30 us; 200 x 1632 x 8128 181 -> 33 us; 315 x 5478 x 11008, float32 out, 4983 -> 60
+// us; 300 x 1000 x 1000 18 -> 9.5 us. Up to 64 rows of W.t() stay on the small-M
+// kernel (16 x 1631 x 8064 164 -> 6.6 us).
 static bool f6_route(int64_t M, int64_t N, int64_t K, int out_dtype, int64_t bsp, int64_t bsn) {
   const bool f32 = out_dtype == QO_DTYPE_F32;
   return (f32 || out_dtype == QO_DTYPE_F16 || out_dtype == QO_DTYPE_BF16) && ((M > 256 && !f32) || ragged(N, K)) &&
